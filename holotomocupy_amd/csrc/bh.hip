@@ -15,6 +15,7 @@
 //               y22 and the shift-gradient partial sums            -> T
 //   K4 object:  gather-form Sadj summed over distances              -> dpsi
 // then the B-spline prefilter of dpsi and two small deterministic reductions.
+#include <algorithm>
 #include <climits>
 
 #include "bh_common.hpp"
@@ -40,6 +41,10 @@ struct BhArgs {
   int accumulate_prb = 0;
   float2* part_r = nullptr;          // [nang*ndist*nz] shift-gradient partials
   double* part_obj = nullptr;        // [column tiles] objective partials
+  float2* part_g = nullptr;          // split angles: [groups <= nang, ndist, nz, n] probe-gradient sums of the
+                                     // groups (NULL: not split)
+  int64_t maxgroups = 0;             // no more groups than this
+  int kper = 0;                      // angles per workgroup of K1
   const float2* twx = nullptr;
   const float2* twy = nullptr;
   const float2* tabx = nullptr;      // [ndist][2][3*(n/2)]
@@ -156,7 +161,10 @@ __device__ __forceinline__ float2 row_sum2(float2 v, float2* red) {
 }
 
 // ---- K1: rows, forward ------------------------------------------------------
-// Workgroup = ROWS row units (j, ty); loops over the angles of the launch.
+// Workgroup = ROWS row units (j, ty) and kper consecutive angles, over which it
+// loops.  The angles are independent: where the row units alone leave the chip
+// idle (256^2 at 2 distances: 64 workgroups for 256 CUs) the host splits them
+// over more workgroups (kFwdBlocks; 684 -> 57 us for 48 angles there).
 // Four waves per SIMD (at most 128 VGPRs): the staged gather waits on memory
 // for about half of its cycles, and the allocator's free choice at N = 2048
 // is 129 registers, i.e. three waves (1.74 against 1.95 ms per 16 angles x 4
@@ -167,7 +175,11 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(4))
   __shared__ float2 lds[ROWS * fft_buf<N>()];
   const int r = threadIdx.x / T, t0 = threadIdx.x % T;
   const int64_t nunits = (int64_t)a.ndist * a.nz;
-  const int64_t unit = xcd_tile(blockIdx.x, gridDim.x) * ROWS + r;  // XCD-contiguous row bands
+  // each XCD takes whole groups of angles (their object planes stay in its L2)
+  const int64_t ublocks = (nunits + ROWS - 1) / ROWS;
+  const int64_t bid = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t unit = bid % ublocks * ROWS + r;
+  const int64_t b0 = bid / ublocks * a.kper, b1 = min(b0 + a.kper, a.nang);
   const bool valid = unit < nunits;
   const int j = valid ? (int)(unit / a.nz) : 0, ty = valid ? (int)(unit % a.nz) : 0;
   float2* s = lds + r * fft_buf<N>();
@@ -175,7 +187,7 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(4))
   fft_load_twiddles<N, E>(twr, t0, a.twx);
   const float2* tab = a.tabx + (int64_t)(j * 2 + 0) * 3 * (N / 2);
   const int64_t plane = (int64_t)a.nzpsi * a.npsi;
-  for (int64_t b = 0; b < a.nang; ++b) {
+  for (int64_t b = b0; b < b1; ++b) {
     // recompute thread-dependent addresses every angle instead of keeping
     // them live across the loop (register pressure)
     int t = t0;
@@ -309,7 +321,42 @@ __global__ __launch_bounds__(C*(N / E)) void bh_cols_k(BhArgs a, int tiles_per_f
 }
 
 // ---- K3: rows, adjoint + epilogue ------------------------------------------
-template <int N, int E, typename TO, bool STAGED>
+// The probe gradient is a sum over the angles of a probe, accumulated per row
+// in LDS, so a workgroup loops over angles.  SPLIT: a workgroup takes a group
+// of at most kAdjGroup consecutive angles and writes its sum to part_g, and
+// bh_prb_final_k adds the groups.  The groups are counted from the first angle
+// of the probe's run, and their size and the use of SPLIT depend on the
+// geometry alone, so the order of the sum, and with it every bit of a request's
+// result, does not depend on what else is in the batch.
+constexpr int kAdjGroup = 4;
+
+// First angle of group q (nang: there are not so many groups).  Every run of
+// equal pidx starts a group, as does every kAdjGroup-th angle of it.  A
+// wavefront step looks at 64 angles; the result is the same in every lane.
+__device__ __forceinline__ int64_t group_start(const int* pidx, int64_t nang, int64_t q) {
+  if (!pidx) return min(q * kAdjGroup, nang);
+  const int lane = threadIdx.x & 63;
+  int64_t run = 0;  // first angle of the run that reaches into this step
+  for (int64_t s0 = 0; s0 < nang; s0 += 64) {
+    const int64_t b = s0 + lane;
+    const bool in = b < nang;
+    const uint64_t heads = __ballot(in && (b == 0 || pidx[b] != pidx[b - 1]));
+    const uint64_t upto = heads & (~0ull >> (63 - lane));  // run heads at or before b
+    const int64_t first = upto ? s0 + 63 - __builtin_clzll(upto) : run;
+    const uint64_t starts = __ballot(in && (b - first) % kAdjGroup == 0);
+    const int count = __builtin_popcountll(starts);
+    if (q < count) {
+      uint64_t rest = starts;
+      for (int64_t k = 0; k < q; ++k) rest &= rest - 1;
+      return s0 + __builtin_ctzll(rest);
+    }
+    q -= count;
+    if (heads) run = s0 + 63 - __builtin_clzll(heads);
+  }
+  return nang;
+}
+
+template <int N, int E, typename TO, bool STAGED, bool SPLIT>
 __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   constexpr int T = N / E, ROWS = kRowThreads / T;
   __shared__ float2 lds[ROWS * fft_buf<N>()];
@@ -317,7 +364,15 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   __shared__ float2 red[kRowThreads / 64];
   const int r = threadIdx.x / T, t0 = threadIdx.x % T;
   const int64_t nunits = (int64_t)a.ndist * a.nz;
-  const int64_t unit = xcd_tile(blockIdx.x, gridDim.x) * ROWS + r;  // XCD-contiguous row bands
+  // XCD-contiguous row bands.  SPLIT: group after group; workgroups without one
+  // are the last ones of the launch (dispatched among the others they would
+  // leave the same shader engines idle each time)
+  const int64_t ublocks = (nunits + ROWS - 1) / ROWS;
+  const int64_t q = SPLIT ? blockIdx.x / ublocks : 0;
+  const int64_t unit = xcd_tile(blockIdx.x - q * ublocks, ublocks) * ROWS + r;
+  const int64_t b0 = SPLIT ? group_start(a.pidx, a.nang, q) : 0;
+  if (b0 >= a.nang) return;  // the whole workgroup
+  const int64_t b1 = SPLIT ? min(b0 + kAdjGroup, a.nang) : a.nang;
   const bool valid = unit < nunits;
   const int j = valid ? (int)(unit / a.nz) : 0, ty = valid ? (int)(unit % a.nz) : 0;
   float2* s = lds + r * fft_buf<N>();
@@ -329,9 +384,17 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   // epilogue and the flushes alike, so no barrier orders them
   float2* acc = lacc + r * N;
   for (int e = 0; e < E; ++e) acc[dct_nat<N>(t0 + e * T)] = make_float2(0.f, 0.f);
-  int pcur = a.pidx ? a.pidx[0] : 0;
+  int pcur = a.pidx ? a.pidx[b0] : 0;
   auto flush = [&](int p) {
     if (!valid) return;
+    if constexpr (SPLIT) {
+      float2* g = a.part_g + ((q * a.ndist + j) * a.nz + ty) * (int64_t)N;
+      for (int e = 0; e < E; ++e) {
+        const int i = dct_nat<N>(t0 + e * T);
+        g[i] = acc[i];
+      }
+      return;
+    }
     float2* g = (a.gprb_p ? a.gprb_p[p] : a.gprb + (int64_t)p * a.ndist * a.nz * N) + ((int64_t)j * a.nz + ty) * N;
     const int t = t0;
     const float rho = a.rho_prb[p];
@@ -343,7 +406,10 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
       acc[i] = make_float2(0.f, 0.f);
     }
   };
-  for (int64_t b = 0; b < a.nang; ++b) {
+  for (int64_t b = b0; b < b1; ++b) {
+    if constexpr (SPLIT) {
+      if (a.pidx && a.pidx[b] != pcur) break;  // the run ends inside the group
+    }
     int t = t0;
     asm volatile("" : "+v"(t));
     const int64_t bj = b * a.ndist + j;
@@ -554,6 +620,31 @@ __global__ __launch_bounds__(256) void bh_pos_final_k(const float2* __restrict__
   }
 }
 
+// Probe gradients of the split K3: per element the group sums of each run of
+// angles in order, then times rho_prb^2 into (or onto) the run's probe.
+__global__ __launch_bounds__(256) void bh_prb_final_k(BhArgs a) {
+  const int64_t field = (int64_t)a.ndist * a.nz * a.n;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= field) return;
+  const float2* part = a.part_g + i;
+  for (int64_t first = 0; first < a.nang;) {
+    const int p = a.pidx ? a.pidx[first] : 0;
+    int64_t end = a.nang;
+    if (a.pidx)
+      for (end = first + 1; end < a.nang && a.pidx[end] == p; ++end) {
+      }
+    float2 tot = make_float2(0.f, 0.f);
+    const int64_t groups = (end - first + kAdjGroup - 1) / kAdjGroup;
+#pragma unroll 4
+    for (int64_t k = 0; k < groups; ++k) tot = cadd(tot, part[k * field]);
+    part += groups * field;
+    float2* g = (a.gprb_p ? a.gprb_p[p] : a.gprb + p * field) + i;
+    const float2 v = cscale(tot, a.rho_prb[p]);
+    *g = a.accumulate_prb ? cadd(*g, v) : v;
+    first = end;
+  }
+}
+
 __global__ __launch_bounds__(256) void bh_sum_k(const double* __restrict__ part, int64_t count,
                                                 double scale, double* __restrict__ out) {
   __shared__ double r[256];
@@ -571,8 +662,25 @@ __global__ __launch_bounds__(256) void bh_sum_k(const double* __restrict__ part,
 // ---- host side --------------------------------------------------------------
 
 struct BhLayout {
-  int64_t c = 0, T = 0, dpsi = 0, part_r = 0, part_obj = 0, total = 0;
+  int64_t c = 0, T = 0, dpsi = 0, part_r = 0, part_obj = 0, part_g = 0, total = 0;
 };
+
+// Workgroups of row units (j, ty) of one angle in the row passes.
+static int64_t row_blocks(int64_t n, int64_t nz, int64_t ndist) {
+  const int64_t rows = n >= 2048 ? 1 : kRowThreads / (n / 8);
+  return (ndist * nz + rows - 1) / rows;
+}
+
+// K3 splits the angles into groups (see there) when one angle's row units are
+// fewer than this (two or three workgroups of it fit a CU, 512 to 768 the chip).
+// 256^2, 2 distances, 48 angles (64 workgroups of row units): 815 -> 149 us and
+// 5 us for bh_prb_final_k; 1024^2 at 3 distances and 16 angles (1536): the whole
+// gradient 1697 against 1697 us; at 2048 and more the extra field of group sums
+// would only cost.
+constexpr int64_t kAdjSplitBelow = 2048;
+static bool adj_split(int64_t n, int64_t nz, int64_t ndist) { return row_blocks(n, nz, ndist) < kAdjSplitBelow; }
+// K1 splits the angles over workgroups until there are about this many.
+constexpr int64_t kFwdBlocks = 4096;
 
 // Column pass of the fused gradient: 16 elements per thread at N = 2048 (two
 // columns per 256-thread workgroup), else 8.
@@ -633,6 +741,8 @@ static BhLayout bh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* sp,
   off += align256(nang * pp->ndist * pp->nz * 8);
   L.part_obj = off;
   off += align256(ntiles * 8);
+  L.part_g = off;
+  if (adj_split(pp->n, pp->nz, pp->ndist)) off += align256(nang * pp->ndist * field * 8);
   L.total = off;
   return L;
 }
@@ -652,20 +762,34 @@ constexpr int bh_row_e() {
 }
 
 template <int N, typename TO>
-static hipError_t launch_rows(bool adjoint, const BhArgs& a, hipStream_t st) {
+static hipError_t launch_rows(bool adjoint, BhArgs a, hipStream_t st) {
   constexpr int E = bh_row_e<N>();
   constexpr int ROWS = kRowThreads / (N / E);
   const int64_t units = (int64_t)a.ndist * a.nz;
-  const int64_t grid = (units + ROWS - 1) / ROWS;
+  const int64_t ublocks = (units + ROWS - 1) / ROWS;
+  const int64_t groups = std::min(a.nang, (kFwdBlocks + ublocks - 1) / ublocks);
+  a.kper = (int)((a.nang + groups - 1) / groups);
+  const bool split = a.part_g != nullptr;
+  const int64_t grid = ublocks * (!adjoint ? (a.nang + a.kper - 1) / a.kper : split ? a.maxgroups : 1);
   const int64_t stat = (int64_t)ROWS * (fft_buf<N>() + (adjoint ? N : 0)) * 8 + 64;
   const int64_t dyn = (int64_t)ROWS * a.npsi * (int64_t)sizeof(TO) * (adjoint ? 2 : 1);
   const bool staged = dyn <= kRowDynBudget && stat + dyn <= kRowLdsBudget;
   if (adjoint) {
-    if (staged)
-      hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, true>), dim3((unsigned)grid), dim3(kRowThreads), (size_t)dyn,
-                         st, a);
+    if (staged && split)
+      hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, true, true>), dim3((unsigned)grid), dim3(kRowThreads),
+                         (size_t)dyn, st, a);
+    else if (staged)
+      hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, true, false>), dim3((unsigned)grid), dim3(kRowThreads),
+                         (size_t)dyn, st, a);
+    else if (split)
+      hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, false, true>), dim3((unsigned)grid), dim3(kRowThreads), 0, st, a);
     else
-      hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, false>), dim3((unsigned)grid), dim3(kRowThreads), 0, st, a);
+      hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, false, false>), dim3((unsigned)grid), dim3(kRowThreads), 0, st,
+                         a);
+    if (split) {
+      const int64_t field = units * N;
+      hipLaunchKernelGGL(bh_prb_final_k, dim3((unsigned)((field + 255) / 256)), dim3(256), 0, st, a);
+    }
   } else {
     if (staged)
       hipLaunchKernelGGL((bh_fwd_rows_k<N, E, TO, true>), dim3((unsigned)grid), dim3(kRowThreads), (size_t)dyn,
@@ -875,6 +999,12 @@ static int bh_gradient_impl(const htamd_bh_plan* p, int64_t nangles, const void*
   a.accumulate_prb = accumulate_prb;
   a.part_r = (float2*)(ws + L.part_r);
   a.part_obj = (double*)(ws + L.part_obj);
+  if (nangles > kAdjGroup && adj_split(a.n, a.nz, a.ndist)) {  // up to one group: the same sum either way
+    a.part_g = (float2*)(ws + L.part_g);
+    // a run ends at most one group early; nprobes is not known without the table
+    const int64_t full = (nangles + kAdjGroup - 1) / kAdjGroup;
+    a.maxgroups = !probe_index ? full : tab && !accumulate_prb ? std::min(nangles, full + nprobes - 1) : nangles;
+  }
   a.twx = p->prop->tw_x;
   a.twy = p->prop->tw_y;
   a.tabx = p->prop->tab_x;

@@ -29,6 +29,7 @@
 //   W0 = dry_y drz_y sum d2wy c - dry_y sum dwy cy - drz_y sum dwy cz
 // so that per pixel  x22 = sum wx R0,  y22 = sum wx Ay - dry_x sum dwx R0,
 //   w22 = dry_x drz_x sum d2wx R0 + sum dwx W1 + sum wx W0.
+#include <algorithm>
 #include <string>
 
 #include "bh_common.hpp"
@@ -79,17 +80,21 @@ struct HessShape {
 // place.  Nothing is held across transforms, so no per-pixel array is kept
 // (the fused form held four or five complex values per pixel across its NF
 // transforms, in scratch).  A workgroup = rpb row units (j, ty) of T = N/E
-// threads; it loops over the angles.  rpb <= kRowThreads / T, chosen so the
-// staged rows fit the dynamic LDS.
+// threads and kper consecutive angles, over which it loops.  rpb <=
+// kRowThreads / T, chosen so the staged rows fit the dynamic LDS.
 template <int N, int E, typename TO, int MODE>
-__global__ __launch_bounds__(kRowThreads) void bhh_chain_k(BhhArgs a, int rpb) {
+__global__ __launch_bounds__(kRowThreads) void bhh_chain_k(BhhArgs a, int rpb, int kper) {
   using HS = HessShape<MODE>;
   constexpr bool SAME = HS::SAME, PAIR = HS::PAIR;
   constexpr int T = N / E;
   constexpr int NR = HS::NR;
   const int r = threadIdx.x / T, t0 = threadIdx.x % T;
   const int64_t nunits = (int64_t)a.ndist * a.nz;
-  const int64_t unit = xcd_tile(blockIdx.x, gridDim.x) * rpb + r;
+  // each XCD takes whole groups of angles (their object planes stay in its L2)
+  const int64_t ublocks = (nunits + rpb - 1) / rpb;
+  const int64_t bid = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t unit = bid % ublocks * rpb + r;
+  const int64_t b0 = bid / ublocks * kper, b1 = min(b0 + kper, a.nang);
   const bool valid = unit < nunits;
   const int j = valid ? (int)(unit / a.nz) : 0, ty = valid ? (int)(unit % a.nz) : 0;
   const int64_t plane = (int64_t)a.nzpsi * a.npsi;
@@ -102,7 +107,7 @@ __global__ __launch_bounds__(kRowThreads) void bhh_chain_k(BhhArgs a, int rpb) {
   TO* V1 = rows + 5 * a.npsi;  // pair: W1 and W0 of the (z, z) form
   TO* V0 = rows + 6 * a.npsi;
   const int64_t prow = ((int64_t)j * a.nz + ty) * N;
-  for (int64_t b = 0; b < a.nang; ++b) {
+  for (int64_t b = b0; b < b1; ++b) {
     int t = t0;
     asm volatile("" : "+v"(t));
     const int64_t bj = b * a.ndist + j;
@@ -513,6 +518,9 @@ static BhhLayout bhh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* s
 // Row pass: 8 elements per thread as the gradient's row passes; the staged
 // rows of a workgroup stay within 64 KiB of dynamic LDS.
 constexpr int64_t kHessDynBudget = 65536;
+// The chain kernel's angles are independent: they are split over workgroups until there are about this many
+// (pair form at 256^2, 4 distances, 32 angles: 781 -> 541 us in all; 1024^2, 16 angles, from 2048: 4539 -> 4351 us).
+constexpr int64_t kHessBlocks = 4096;
 
 template <int N, typename TO, int MODE>
 static hipError_t hess_rows_m(const BhhArgs& a, hipStream_t st) {
@@ -522,9 +530,12 @@ static hipError_t hess_rows_m(const BhhArgs& a, hipStream_t st) {
   int rpb = ROWS;
   while (rpb > 1 && rpb * per_row > kHessDynBudget) rpb >>= 1;
   if (rpb * per_row > kHessDynBudget) return hipErrorInvalidConfiguration;
-  const int64_t grid = ((int64_t)a.ndist * a.nz + rpb - 1) / rpb;
+  const int64_t ublocks = ((int64_t)a.ndist * a.nz + rpb - 1) / rpb;
+  const int64_t groups = std::min(a.nang, (kHessBlocks + ublocks - 1) / ublocks);
+  const int64_t kper = (a.nang + groups - 1) / groups;
+  const int64_t grid = ublocks * ((a.nang + kper - 1) / kper);
   hipLaunchKernelGGL((bhh_chain_k<N, E, TO, MODE>), dim3((unsigned)grid), dim3(rpb * T), (size_t)(rpb * per_row),
-                     st, a, rpb);
+                     st, a, rpb, (int)kper);
   return hipGetLastError();
 }
 

@@ -220,3 +220,56 @@ def test_fused_gradient_bench_size_properties(gpu):
         rec.gradients_fused(part, out, data[st:st + 2], st=st)
     assert torch.equal(gs["proj"], g1["proj"]) and torch.equal(gs["pos"], g1["pos"])
     assert rel(gs["prb"], g1["prb"].cpu().numpy()) < 1e-6
+
+
+@pytest.mark.parametrize("n,ndist,runs", [(64, 2, (1, 4, 5, 9, 3)), (128, 3, (70, 1, 8))])
+def test_probe_runs_alone_and_together(gpu, n, ndist, runs):
+    """Groups of angles whose probe-gradient sums are formed apart and added:
+    runs shorter than, equal to and longer than a group (and than the 64
+    angles that one look back covers) give the same bits alone and in one
+    launch, and the per-operator cascade's gradient."""
+    print(f"[case] probe runs n={n} ndist={ndist} runs={runs}", flush=True)
+    from holotomocupy_amd.bh import BHGradient
+    B = sum(runs)
+    rec, cas, x, v, w, d = make_problem(False, n=n, nobj=48, ndist=ndist, B=B, seed=61)
+    xd, dd = dev(x), torch.from_numpy(d).cuda()
+    bh = BHGradient(rec)
+    mag = rec.eff_demagnifications[:B].contiguous()
+    k = len(runs)
+    prb = torch.stack([xd["prb"] * (1 + 0.1 * i) for i in range(k)]).contiguous()
+    pidx = torch.tensor(sum(([i] * m for i, m in enumerate(runs)), []), dtype=torch.int32, device="cuda")
+    s, rp = bh.scales(B)
+    gproj, gpos, gprb = torch.empty_like(xd["proj"]), torch.empty_like(xd["pos"]), torch.empty_like(prb)
+    bh(prb, xd["proj"], xd["pos"], dd, mag, gproj, gpos, gprb, accumulate_prb=False, probe_index=pidx, scales=s,
+       rho_prb=rp.repeat(k))
+    st = 0
+    for i, m in enumerate(runs):
+        sl = slice(st, st + m)
+        one = {"prb": torch.zeros_like(xd["prb"]), "proj": torch.empty_like(gproj[sl]),
+               "pos": torch.empty_like(gpos[sl])}
+        var = {"prb": prb[i], "proj": xd["proj"][sl], "pos": xd["pos"][sl]}
+        rec.gradients_fused(var, one, dd[sl], st=st)
+        assert torch.equal(one["prb"], gprb[i]), i
+        assert torch.equal(one["proj"], gproj[sl]) and torch.equal(one["pos"], gpos[sl]), i
+        ref = {q: torch.zeros_like(t) for q, t in one.items()}
+        rec.gradients_cascade(var, ref, dd[sl], st=st)
+        assert rel(one["prb"], ref["prb"].cpu().numpy()) < 1e-5
+        st += m
+
+
+def test_angles_split_over_workgroups_with_a_remainder(gpu):
+    """More angles than the row passes have workgroups for: each workgroup
+    takes two, the last one one."""
+    print("[case] row passes with two angles per workgroup", flush=True)
+    B = 35
+    rec, cas, x, v, w, d = make_problem(False, n=256, nobj=48, ndist=4, B=B, seed=62)
+    xd, yd, dd = dev(x), dev(v), torch.from_numpy(d).cuda()
+    g, ref = ({q: torch.zeros_like(t) for q, t in xd.items()} for _ in range(2))
+    rec.gradients_fused(xd, g, dd)
+    rec.gradients_cascade(xd, ref, dd)
+    assert rel(g["prb"], ref["prb"].cpu().numpy()) < 1e-5
+    assert rel(g["proj"], ref["proj"].cpu().numpy()) < 1e-5
+    assert rel(g["pos"], ref["pos"].cpu().numpy()) < 1e-4
+    for z in (yd, dev(w)):
+        h = rec.hessian_fused(xd, yd, yd if z is yd else z, dd).item()
+        assert h == pytest.approx(rec.hessian_cascade(xd, yd, yd if z is yd else z, dd), rel=1e-4)

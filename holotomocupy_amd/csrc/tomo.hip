@@ -9,10 +9,10 @@
 // non-zero rows of the embedded slice are transformed along x), with the sign
 // modulations, zero-embedding, cropping and deapodisation folded into the
 // loads and stores.  The 9x9 Gaussian gridding taps of every polar sample are
-// built once per plan in FP64 (stored FP32): the forward gathers them per
-// (angle, slice) line with the line's 1-D FFT fused; the adjoint uses the same
-// taps transposed (one CSR row per grid point) and gathers onto the grid from
-// a slice-contiguous copy of the transformed sinogram -- the reference's atomic
+// built once per plan in FP64 (stored FP32): the forward gathers them through
+// LDS tiles of the grid; the adjoint sorts the samples by 4x4 tile of the grid
+// and forms each tile as a matrix product over its samples, from a
+// slice-contiguous copy of the transformed sinogram -- the reference's atomic
 // scatter in a fixed summation order.
 #include <algorithm>
 #include <cmath>
@@ -33,12 +33,15 @@ struct TomoArgs {
   const float* phi = nullptr;      // [n, n] deapodisation (mask and scale included)
   const float2* tw2 = nullptr;     // twiddles of length 2n
   const float2* tw1 = nullptr;     // twiddles of length n
-  // gridding taps of polar sample s = theta n + t (built in FP64 on the host):
-  const int2* tb = nullptr;        // [ntheta n] first tap (bx, by) on the 2n grid, before wrapping
-  const float* tw = nullptr;       // [2L][ntheta n]: wx[i] at tw[i S + s], wy[i] at tw[(L + i) S + s]
-  // the same taps transposed, one row per grid point g = row 2n + col (CSR):
-  const int* rp = nullptr;         // [4 n^2 + 1]
-  const int2* csw = nullptr;       // [nnz] (sample index s, weight wy wx as float bits)
+  // gridding taps of polar sample s = theta n + t, built in FP64 on the host:
+  // weights along x at wt[2 kWRow s + 3 + i] and along y at wt[2 kWRow s +
+  // kWRow + 3 + i], tap i < 9, zero elsewhere
+  const float* wt = nullptr;
+  // the samples by tile of 4x4 grid points: entries [tp[t], tp[t + 1]) of tile
+  // t = row n / 2 + column touch it, each (sample, oy << 8 | ox) with ox the
+  // index in the sample's x weights of the tile's first column (oy of its row)
+  const int* tp = nullptr;
+  const int2* te = nullptr;
   // the samples binned by grid tile for the forward gather: work item i covers
   // samples [it.z, it.z + it.w) of the sorted list, all in tile (it.x, it.y);
   // per sorted sample: (local tap origin oy << 16 | ox, sample index) and the
@@ -52,10 +55,9 @@ struct TomoArgs {
   float2* W = nullptr;             // [nz, n, 2n]
   float2* G = nullptr;             // [nz, 2n, 2n]
   float2* Sh = nullptr;            // [ntheta n, nz] transformed sinogram (RT)
-  // grid points whose CSR rows are longer than kHeavyRow, longest first; the
-  // thread-per-point gather skips them and a wavefront per point sums them
-  const int* heavy = nullptr;
+  const int* heavy = nullptr;      // tiles with more than kHeavyTile entries, longest first
   int nheavy = 0;
+  int longest = 0;                 // entries of the longest list
   // per-bin factor of the adjoint's line transform (NULL = none): the
   // detector filter of filtered back-projection, shifted by n/2 to the bins
   // of the c1d-modulated transform and scaled by sqrt(n / ntheta)
@@ -136,55 +138,6 @@ __global__ __launch_bounds__(C*(N2 / E)) void tomo_cols_fwd_k(TomoArgs a) {
     const int idx = threadIdx.x + e * NT;
     const int c = idx % C, k = idx / C;
     dst[k * N2 + c] = cscale(lds[c * LS + fpad(k)], sgnf(k));
-  }
-}
-
-// ---- forward pass C: gather + line IFFT ------------------------------------
-template <int N, int E, typename TO>
-__global__ __launch_bounds__(256) void tomo_gather_k(TomoArgs a, TO* __restrict__ out) {
-  constexpr int T = N / E, ROWS = 256 / T;
-  __shared__ float2 lds[ROWS * fft_buf<N>()];
-  const int r = threadIdx.x / T, t = threadIdx.x % T;
-  const int64_t line = (int64_t)blockIdx.x * ROWS + r;  // (theta, z)
-  const bool valid = line < (int64_t)a.ntheta * a.nz;
-  const int th = valid ? (int)(line / a.nz) : 0;
-  const int z = valid ? (int)(line % a.nz) : 0;
-  float2* s = lds + r * fft_buf<N>();
-  FftTw<N, E> twr;
-  fft_load_twiddles<N, E>(twr, t, a.tw1);
-  const int n2 = 2 * N;
-  const float2* g = a.G + (int64_t)z * n2 * n2;
-  const int L = 2 * a.m + 1;
-  const int64_t S = (int64_t)a.ntheta * N;
-  for (int e = 0; e < E; ++e) {
-    const int tt = t + e * T;
-    const int64_t si = (int64_t)th * N + tt;
-    const int2 b = a.tb[si];
-    const int bx = b.x, by = b.y;
-    float wx[16];
-    for (int i0 = 0; i0 < L; ++i0) wx[i0] = a.tw[i0 * S + si];
-    float2 acc = make_float2(0.f, 0.f);
-    for (int i1 = 0; i1 < L; ++i1) {
-      const float wy = a.tw[(L + i1) * S + si];
-      const int row = (N + by + i1 + n2) % n2;
-      float2 racc = make_float2(0.f, 0.f);
-      for (int i0 = 0; i0 < L; ++i0) {
-        const int col = (N + bx + i0 + n2) % n2;
-        racc = vfma(wx[i0], g[(int64_t)row * n2 + col], racc);
-      }
-      acc = vfma(wy, racc, acc);
-    }
-    // c1d . (gather / n), c1d[k] = (-1)^(k+1)
-    s[fpad(tt)] = cscale(acc, -sgnf(tt) / (float)N);
-  }
-  __syncthreads();
-  fft_lds<N, E, true>(s, t, twr);
-  if (valid) {
-    TO* dst = out + ((int64_t)th * a.nz + z) * N;
-    for (int e = 0; e < E; ++e) {
-      const int tt = t + e * T;
-      st_c<TO>(dst, tt, cscale(s[fpad(tt)], -sgnf(tt) / (4.0f * N)));
-    }
   }
 }
 
@@ -362,141 +315,222 @@ __global__ __launch_bounds__(256) void tomo_filter_k(const TIO* in, TIO* out, in
   }
 }
 
-// ---- adjoint pass C'': gather onto the grid (transpose of the forward taps) ---
-// Grid point g sums w_k Sh[s_k, z] over its CSR row (packed 8-byte (sample,
-// weight) pairs) in entry order: deterministic, no atomics.  The lanes of a
-// wavefront run across ZB consecutive slices of P = 64 / ZB points, so one
-// entry of a point is one (wave-uniform for ZB = 64) index load and one
-// contiguous ZB x 8-byte read of the sample's slice block -- every byte of a
-// fetched line is used by the instruction that fetched it.  Entries are taken
-// kGatherBatch at a time so that many independent reads are in flight.
-//
-// A workgroup (4 wavefronts) owns PT consecutive grid points and ZB slices;
-// its results go through an LDS tile so the grid is written as rows of PT
-// points per slice (PT = 32, more where a wave step takes 64 / ZB > 8 points;
-// 64 points, LDS-bound at 4 workgroups per CU, measured 9% slower).  Rows through the centre of the grid collect a
-// sample of every angle (at 256^2 with 384 angles the longest has 2005
-// entries against a mean of 30): rows longer than kHeavyRow entries are left
-// to tomo_grid_gather_heavy_k, launched after this kernel on the same stream,
-// which overwrites those points.
-constexpr int kHeavyRow = 64;
-constexpr int kGatherBatch = 8;
-constexpr int kGatherPoints = 32;  // grid points per workgroup of the light rows (at least 4 wave steps)
-constexpr int kHeavyWaves = 4;     // wavefronts per heavy row
+// ---- adjoint pass C'': samples onto the grid --------------------------------
+// G[g][z] = sum over the samples s whose 9x9 window covers grid point g of
+// wy(s, g) wx(s, g) Sh[s][z]: for one tile of 4x4 points the product of a
+// 16 x K matrix of weights (K samples touch the tile, about 9/4 of their
+// weights are not zero) with K rows of slices, which is what the matrix
+// instructions do: v_mfma_f32_16x16x4_f32 takes four samples at a time, the
+// tile's points as rows and 16 floats of slices as columns, FP32 throughout.
+// Against a sum per point, a sample's slices are read by the 9 tiles it
+// touches instead of by 81 points; those reads (from L2) bounded the gather.
+// A wavefront owns one tile and 16 VEC U slices.  Lane l holds sample l / 16
+// of the four, reads its VEC slices at q = l % 16 (their re and im columns are
+// separate products, so 2 VEC U accumulators) and forms the weight of point
+// l % 16 from the sample's two zero-padded weight rows (built in FP64).  The
+// order of each sum is the list's, whatever runs when; no atomics.
+// The four wavefronts of a workgroup take four tiles of a row, which share most
+// of their samples and make whole cache lines of the result.  Every line crosses the centre, so the lists there are long (2500
+// samples at 256^2, 384 angles, against a mean of 54): the tiles with more
+// than kHeavyTile entries (listed longest first, at the front of the launch)
+// take a whole workgroup, which cuts the list in four and adds the four sums
+// in order.
+// 256 slices of 256^2, 384 angles: 1555 us with a sum per point -> 390 us (1.2 GB
+// through the L2 misses, a third of it the grid; the products themselves are 104 us);
+// 45 real slices of 512^2, 451 angles (filtered back-projection): 1645 -> 275 us.
+constexpr int kHeavyTile = 128;
+constexpr int kLongTile = 512;  // from here more wavefronts share a long list (few slices)
+constexpr int kBatch = 4;  // steps of four samples taken together
+constexpr int kWRow = 16;  // a sample's weights along an axis: 3 zeros, 9 taps, 4 zeros
 
-template <int ZB>
-constexpr int gather_points() {
-  return kGatherPoints > 4 * (64 / ZB) ? kGatherPoints : 4 * (64 / ZB);
-}
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(8)));  // an odd slice count leaves rows 8-byte aligned
 
-// acc += sum over entries [k0, k1) of w Sh[s, z] in entry order, for the
-// slice block starting at src = Sh + z (zin: this lane's slice exists)
-__device__ __forceinline__ float2 gather_entries(const int2* __restrict__ csw, const float2* __restrict__ src,
-                                                 int64_t nz, int k0, int k1, bool zin, float2 acc) {
-  int k = k0;
-  for (; k + kGatherBatch <= k1; k += kGatherBatch) {
-    int2 cw[kGatherBatch];
-    float2 v[kGatherBatch];
-#pragma unroll
-    for (int u = 0; u < kGatherBatch; ++u) cw[u] = csw[k + u];
-#pragma unroll
-    for (int u = 0; u < kGatherBatch; ++u) v[u] = zin ? src[(int64_t)cw[u].x * nz] : make_float2(0.f, 0.f);
-#pragma unroll
-    for (int u = 0; u < kGatherBatch; ++u) acc = vfma(__int_as_float(cw[u].y), v[u], acc);
-  }
-  for (; k < k1; ++k) {
-    const int2 cw = csw[k];
-    const float2 v = zin ? src[(int64_t)cw.x * nz] : make_float2(0.f, 0.f);
-    acc = vfma(__int_as_float(cw.y), v, acc);
-  }
-  return acc;
-}
-
-template <int ZB, bool FULL>
-__global__ __launch_bounds__(256) void tomo_grid_gather_k(TomoArgs a) {
-  constexpr int P = 64 / ZB, PT = gather_points<ZB>(), TS = PT + 1;  // points per wave step, per workgroup; tile stride
-  static_assert(PT % (4 * P) == 0, "whole wave steps per workgroup");
-  __shared__ float2 tile[ZB * TS];
-  const int64_t n4 = 4LL * a.n * a.n;
-  const int64_t g0 = (int64_t)blockIdx.x * PT;
-  const int z0 = blockIdx.y * ZB;
+template <int VEC, int U, int NW>
+__global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
+  constexpr int NA = 2 * VEC * U;  // accumulators: float columns of 16 slices
+  constexpr int PX = 4 * NW;       // points of a workgroup's row
+  constexpr int ZS = 4 * PX + 2;   // float2 slots of a slice's 4 rows, padded off its bank
+  constexpr int kOut = 16 * VEC * U * ZS / 2, kPart = (NW - 1) * NA * 64;
+  __shared__ f32x4 lds[kOut > kPart ? kOut : kPart];
+  __shared__ int skipped[NW];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
-  const int ps = lane / ZB, q = lane % ZB;
-  const bool zin = FULL || z0 + q < a.nz;
-  const float2* src = a.Sh + z0 + q;
-#pragma unroll 1
-  for (int it = 0; it < PT / 4 / P; ++it) {
-    const int pl = wv * (PT / 4) + it * P + ps;  // point of the tile
-    const int64_t g = g0 + pl;
-    float2 acc = make_float2(0.f, 0.f);
-    if (g < n4) {
-      const int k0 = a.rp[g], k1 = a.rp[g + 1];
-      if (k1 - k0 <= kHeavyRow) acc = gather_entries(a.csw, src, a.nz, k0, k1, zin, acc);
+  const int q = lane & 15, kk = lane >> 4;
+  const int nt = a.n / 2, n2 = 2 * a.n;
+  const bool heavy = (int)blockIdx.x < a.nheavy;
+  bool skip = false;  // nothing of this wavefront's is stored
+  int tile, beg, end;
+  if (heavy) {
+    tile = a.heavy[blockIdx.x];
+    const int b = a.tp[tile], steps = (a.tp[tile + 1] - b) / 4;
+    beg = b + steps * wv / NW * 4;
+    end = b + steps * (wv + 1) / NW * 4;
+  } else {
+    const int nb = (nt + NW - 1) / NW;
+    const int bid = (int)xcd_tile(blockIdx.x - a.nheavy, gridDim.x - a.nheavy);
+    const int tx = bid % nb * NW + wv;
+    tile = bid / nb * nt + min(tx, nt - 1);
+    beg = a.tp[tile];
+    end = a.tp[tile + 1];
+    skip = tx >= nt || end - beg > kHeavyTile;
+    if (skip) end = beg;
+  }
+  const int z0 = blockIdx.y * zper, z1 = min(z0 + zper, a.nz);
+  int zc[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) zc[u] = min(z0 + (u * 16 + q) * VEC, a.nz - VEC);
+  const float* wt = a.wt + (q & 3);
+  const float* wty = a.wt + kWRow + (q >> 2);
+  // the running sum rounds at every step: sums of kBatch steps, added up, keep
+  // the error of the longest lists at that of the shortest (RT at 256^2 and 720
+  // angles against FP64: 8.2e-7 in one sum, 2.3e-7 so, 2.4e-7 with a sum per
+  // point)
+  f32x4 tot[NA];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) tot[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // a batch's entries are loaded a batch ahead, one per lane, and its samples'
+  // slices and weights all at once; entries past the end repeat the last with
+  // zero weight (as the lists' padding to whole steps has)
+  int2 next = make_int2(0, 0);
+  auto entries = [&](int e) { next = a.te[min(e + (lane & (4 * kBatch - 1)), end - 1)]; };
+  auto load = [&](int e, float (&w)[kBatch], float (&v)[kBatch][U][2 * VEC]) {
+    const int2 cur = next;
+    entries(e + 4 * kBatch);
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int s = __shfl(cur.x, 4 * i + kk, 64), o = __shfl(cur.y, 4 * i + kk, 64);
+      const int64_t ws = (int64_t)s * (2 * kWRow);
+      w[i] = e + 4 * i < end ? wt[ws + (o & 0xff)] * wty[ws + (o >> 8)] : 0.f;
+      const float2* src = a.Sh + (int64_t)s * a.nz;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if constexpr (VEC == 2) {
+          const f32x4u t = *reinterpret_cast<const f32x4u*>(src + zc[u]);
+          v[i][u][0] = t.x; v[i][u][1] = t.y; v[i][u][2] = t.z; v[i][u][3] = t.w;
+        } else {
+          const float2 t = src[zc[u]];
+          v[i][u][0] = t.x; v[i][u][1] = t.y;
+        }
+      }
     }
-    tile[q * TS + pl] = acc;
-  }
-  __syncthreads();
-  // slice r of the tile is PT consecutive grid points, written contiguously
+  };
+  auto mul = [&](const float (&w)[kBatch], const float (&v)[kBatch][U][2 * VEC]) {
+    f32x4 acc[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < 2 * VEC; ++c)
+          acc[u * 2 * VEC + c] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], v[i][u][c], acc[u * 2 * VEC + c], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) tot[i] += acc[i];
+  };
+  if (beg < end) {
+    float w0[kBatch], v0[kBatch][U][2 * VEC];
+    entries(beg);
+    if constexpr (NA <= 4) {
+      // few slices: a wavefront's chain of loads is what counts, so two batches
+      // take turns, one loading while the other is multiplied (with more
+      // slices the second set of registers costs more wavefronts than it gains)
+      float w1[kBatch], v1[kBatch][U][2 * VEC];
+      load(beg, w0, v0);
 #pragma unroll 1
-  for (int i = threadIdx.x; i < ZB * PT; i += 256) {
-    const int r = i / PT, pl = i % PT;
-    const int64_t g = g0 + pl;
-    if (g < n4 && (FULL || z0 + r < a.nz)) a.G[(int64_t)(z0 + r) * n4 + g] = tile[r * TS + pl];
+      for (int e = beg;; e += 8 * kBatch) {
+        const bool more1 = e + 4 * kBatch < end, more2 = e + 8 * kBatch < end;
+        if (more1) load(e + 4 * kBatch, w1, v1);
+        mul(w0, v0);
+        if (!more1) break;
+        if (more2) load(e + 8 * kBatch, w0, v0);
+        mul(w1, v1);
+        if (!more2) break;
+      }
+    } else {
+#pragma unroll 1
+      for (int e = beg; e < end; e += 4 * kBatch) {
+        load(e, w0, v0);
+        mul(w0, v0);
+      }
+    }
   }
-}
-
-// One workgroup per heavy grid point and ZB slices: its NC = kHeavyWaves P
-// lane groups each sum one contiguous chunk of the point's entries (chunk
-// c = wave P + group, entries [k0 + c L / NC, k0 + (c + 1) L / NC)), in entry order, and lane q
-// then adds the chunks' sums for slice q in chunk order -- a fixed order, so
-// the result does not depend on scheduling.
-template <int ZB, bool FULL>
-__global__ __launch_bounds__(64 * kHeavyWaves) void tomo_grid_gather_heavy_k(TomoArgs a) {
-  constexpr int P = 64 / ZB, NC = kHeavyWaves * P;
-  __shared__ float2 part[NC * ZB];
-  const int64_t n4 = 4LL * a.n * a.n;
-  const int g = a.heavy[blockIdx.x];
-  const int z0 = blockIdx.y * ZB;
-  const int wv = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int ps = lane / ZB, q = lane % ZB;
-  const bool zin = FULL || z0 + q < a.nz;
-  const int k0 = a.rp[g], L = a.rp[g + 1] - k0;
-  const int c = wv * P + ps;
-  const int kb = k0 + (int)((int64_t)L * c / NC), ke = k0 + (int)((int64_t)L * (c + 1) / NC);
-  part[c * ZB + q] = gather_entries(a.csw, a.Sh + z0 + q, a.nz, kb, ke, zin, make_float2(0.f, 0.f));
+  const int64_t plane = (int64_t)n2 * n2;
+  if (heavy) {
+    f32x4(*part)[NA][64] = reinterpret_cast<f32x4(*)[NA][64]>(lds);
+    if (wv) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) part[wv - 1][i][lane] = tot[i];
+    }
+    __syncthreads();
+    if (wv) return;
+#pragma unroll
+    for (int k = 0; k < NW - 1; ++k)
+#pragma unroll
+      for (int i = 0; i < NA; ++i) tot[i] += part[k][i][lane];
+    float2* dst = a.G + (int64_t)(tile / nt * 4 + kk) * n2 + tile % nt * 4;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) {
+        if (z0 + (u * 16 + q) * VEC >= z1) continue;
+        const f32x4 re = tot[(u * VEC + c) * 2], im = tot[(u * VEC + c) * 2 + 1];
+        float2* d = dst + (zc[u] + c) * plane;
+        *reinterpret_cast<f32x4u*>(d) = f32x4{re.x, im.x, re.y, im.y};
+        *reinterpret_cast<f32x4u*>(d + 2) = f32x4{re.z, im.z, re.w, im.w};
+      }
+    return;
+  }
+  // result rows 4 (l / 16) + r are the points (y = l / 16, x = r), columns q
+  // the slices: through LDS, so that a slice's row is stored as whole lines
+  float2* out = reinterpret_cast<float2*>(lds);
+  if (lane == 0) skipped[wv] = skip;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) {
+      const f32x4 re = tot[(u * VEC + c) * 2], im = tot[(u * VEC + c) * 2 + 1];
+      const int slot = zc[u] + c - z0;  // lanes past the last slice repeat it
+      if (slot < 0) continue;
+      f32x4* d = reinterpret_cast<f32x4*>(out + slot * ZS + kk * PX + wv * 4);
+      d[0] = f32x4{re.x, im.x, re.y, im.y};
+      d[1] = f32x4{re.z, im.z, re.w, im.w};
+    }
   __syncthreads();
-  if (threadIdx.x < ZB && (FULL || z0 + (int)threadIdx.x < a.nz)) {
-    float2 t = make_float2(0.f, 0.f);
-    for (int cc = 0; cc < NC; ++cc) t = cadd(t, part[cc * ZB + threadIdx.x]);
-    a.G[(int64_t)(z0 + threadIdx.x) * n4 + g] = t;
+  const int tx0 = tile % nt / NW * NW, gy = tile / nt * 4;  // the workgroup's first tile (tile is clamped to its row)
+  constexpr int TR = PX / 2;                                 // threads of a row, 2 points each
+  const int t = threadIdx.x % TR;
+  if (skipped[t >> 1]) return;
+  for (int r = threadIdx.x / TR; r < 4 * (z1 - z0); r += 64 * NW / TR) {
+    const int zl = r >> 2, y = r & 3;
+    // not kept in the L2: the samples' slices, which the next tiles read, are
+    // (787 -> 736 us)
+    __builtin_nontemporal_store(
+        *reinterpret_cast<const f32x4u*>(out + zl * ZS + y * PX + t * 2),
+        reinterpret_cast<f32x4u*>(a.G + (z0 + zl) * plane + (int64_t)(gy + y) * n2 + tx0 * 4 + t * 2));
   }
 }
 
-// The grid gather of the adjoint: the rows up to kHeavyRow entries, then the
-// heavy rows.  ZB = 64 slices per workgroup where they divide the slab, else
-// 32, 16, or 8 with the last block masked.
-template <int ZB, bool FULL>
-static void launch_grid_gather_zb(const TomoArgs& a, hipStream_t st) {
-  const int64_t n4 = 4LL * a.n * a.n;
-  const unsigned zb = (unsigned)((a.nz + ZB - 1) / ZB);
-  constexpr int PT = gather_points<ZB>();
-  hipLaunchKernelGGL((tomo_grid_gather_k<ZB, FULL>), dim3((unsigned)((n4 + PT - 1) / PT), zb), dim3(256), 0, st, a);
-  if (a.nheavy)
-    hipLaunchKernelGGL((tomo_grid_gather_heavy_k<ZB, FULL>), dim3((unsigned)a.nheavy, zb), dim3(64 * kHeavyWaves), 0,
-                       st, a);
-}
-
+// Slices a wavefront takes: the smallest of 16, 32, 48 and 64 that holds an
+// even share of the slab (a share ends anywhere: a lane past the end repeats
+// the last slices).
 static hipError_t launch_grid_gather(const TomoArgs& a, hipStream_t st) {
-  if (a.nz % 64 == 0)
-    launch_grid_gather_zb<64, true>(a, st);
-  else if (a.nz % 32 == 0)
-    launch_grid_gather_zb<32, true>(a, st);
-  else if (a.nz % 16 == 0)
-    launch_grid_gather_zb<16, true>(a, st);
-  else if (a.nz % 8 == 0)
-    launch_grid_gather_zb<8, true>(a, st);
+  const int nt = a.n / 2;
+  const int zblocks = (a.nz + 63) / 64, zper = ((a.nz + zblocks - 1) / zblocks + 1) / 2 * 2;
+  auto grid = [&](int nw) { return dim3((unsigned)(a.nheavy + (nt + nw - 1) / nw * nt), (unsigned)zblocks); };
+  if (zper <= 16 && a.longest > kLongTile)
+    hipLaunchKernelGGL((tomo_grid_k<1, 1, 16>), grid(16), dim3(1024), 0, st, a, zper);
+  else if (zper <= 16)
+    hipLaunchKernelGGL((tomo_grid_k<1, 1, 4>), grid(4), dim3(256), 0, st, a, zper);
+  else if (zper <= 32 && a.longest > kLongTile)
+    hipLaunchKernelGGL((tomo_grid_k<2, 1, 8>), grid(8), dim3(512), 0, st, a, zper);
+  else if (zper <= 32)
+    hipLaunchKernelGGL((tomo_grid_k<2, 1, 4>), grid(4), dim3(256), 0, st, a, zper);
+  else if (zper <= 48)
+    hipLaunchKernelGGL((tomo_grid_k<1, 3, 4>), grid(4), dim3(256), 0, st, a, zper);
   else
-    launch_grid_gather_zb<8, false>(a, st);
+    hipLaunchKernelGGL((tomo_grid_k<2, 2, 4>), grid(4), dim3(256), 0, st, a, zper);
   return hipGetLastError();
 }
 
@@ -693,7 +727,7 @@ static bool tomo_any_ffts(const TomoArgs& a, AnyFft* f2, AnyFft* f1) {
 template <typename TIO>
 static hipError_t tomo_fwd_any(const TomoArgs& a, const TIO* obj, TIO* out, hipStream_t st) {
   AnyFft f2, f1;
-  if (!tomo_any_ffts(a, &f2, &f1) || !a.items) return hipErrorInvalidValue;
+  if (!tomo_any_ffts(a, &f2, &f1)) return hipErrorInvalidValue;
   const int N2 = 2 * a.n;
   hipError_t e = any_launch_rows(TomoRowsFwdAny<TIO>{a, obj}, f2, (int64_t)a.nz * a.n, st);
   if (e != hipSuccess) return e;
@@ -746,16 +780,11 @@ static hipError_t tomo_fwd_n(const TomoArgs& a, const TIO* obj, TIO* out, hipStr
   constexpr int EL = N >= 8 ? 8 : N;
   constexpr int RL = 256 / (N / EL);
   const int64_t lines = (int64_t)a.ntheta * a.nz;
-  if (a.items) {
-    hipLaunchKernelGGL(tomo_tile_gather_k, dim3((unsigned)a.nitems, (unsigned)((a.nz + kTZ - 1) / kTZ)), dim3(256),
-                       0, st, a);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL((tomo_line_ifft_k<N, EL, TIO>), dim3((unsigned)((lines + RL - 1) / RL)), dim3(256), 0, st, a,
-                       out);
-  } else {
-    hipLaunchKernelGGL((tomo_gather_k<N, EL, TIO>), dim3((unsigned)((lines + RL - 1) / RL)), dim3(256), 0, st, a,
-                       out);
-  }
+  hipLaunchKernelGGL(tomo_tile_gather_k, dim3((unsigned)a.nitems, (unsigned)((a.nz + kTZ - 1) / kTZ)), dim3(256), 0,
+                     st, a);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  hipLaunchKernelGGL((tomo_line_ifft_k<N, EL, TIO>), dim3((unsigned)((lines + RL - 1) / RL)), dim3(256), 0, st, a,
+                     out);
   return hipGetLastError();
 }
 
@@ -838,15 +867,14 @@ struct htamd_tomo_plan {
   float* phi = nullptr;
   float2* tw2 = nullptr;
   float2* tw1 = nullptr;
-  int2* tb = nullptr;
-  float* tw = nullptr;
-  int* rp = nullptr;
-  int2* csw = nullptr;
+  float* wt = nullptr;
+  int* tp = nullptr;
+  int2* te = nullptr;
   int4* items = nullptr;
   int2* so = nullptr;
   float2* sf = nullptr;
   int* heavy = nullptr;
-  int nitems = 0, ts = 0, nheavy = 0;
+  int nitems = 0, ts = 0, nheavy = 0, longest = 0;
   // detector filters (ramp, Shepp-Logan, Parzen): [3][n] with the 1/n of the
   // inverse transform for htamd_tomo_filter, and [3][n] shifted by n/2 and
   // scaled by sqrt(n / ntheta) for htamd_tomo_fbp
@@ -898,9 +926,9 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
   const double eps = 1e-3;
   p->mu = -std::log(eps) / (2.0 * (double)n * (double)n);
   p->m = (int)std::ceil(2.0 * n / M_PI * std::sqrt(-p->mu * std::log(eps) + (p->mu * n) * (p->mu * n) / 4.0));
-  if (p->m > 7) {
+  if (2 * p->m + 1 != kTL) {  // 4 for every n: the kernels are built for 9x9 windows
     delete p;
-    return fail(HTAMD_ERR_UNSUPPORTED, "tomo_plan_create: gridding half-width above 7");
+    return fail(HTAMD_ERR_UNSUPPORTED, "tomo_plan_create: gridding half-width is not 4");
   }
   const int L = 2 * p->m + 1;
   const int64_t S = ntheta * n, n2 = 2 * n;
@@ -914,7 +942,7 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
   // x0 = (t - n/2) cos / n, y0 = -(t - n/2) sin / n, first tap floor(2n x0) - m,
   // weights exp(-pi^2/mu d^2) (x) and pi/mu exp(-pi^2/mu d^2) (y).
   std::vector<int2> tb((size_t)S);
-  std::vector<float> tw((size_t)(2 * L * S));
+  std::vector<float> wt((size_t)(2 * kWRow * S), 0.0f);
   const double cy = M_PI / p->mu, cx = -M_PI * M_PI / p->mu, inv2n = 1.0 / (double)n2;
   for (int64_t k = 0; k < ntheta; ++k) {
     const double th = (double)(float)theta[k];
@@ -926,44 +954,43 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
       const int bx = (int)std::floor((double)n2 * x0) - p->m;
       const int by = (int)std::floor((double)n2 * y0) - p->m;
       tb[(size_t)si] = make_int2(bx, by);
+      float* w = &wt[(size_t)(2 * kWRow * si)];
       for (int i = 0; i < L; ++i) {
         const double dx = (bx + i) * inv2n - x0, dy = (by + i) * inv2n - y0;
-        tw[(size_t)(i * S + si)] = (float)std::exp(cx * dx * dx);
-        tw[(size_t)((L + i) * S + si)] = (float)(cy * std::exp(cx * dy * dy));
+        w[3 + i] = (float)std::exp(cx * dx * dx);
+        w[kWRow + 3 + i] = (float)(cy * std::exp(cx * dy * dy));
       }
     }
   }
-  // The same taps grouped by grid point (CSR, counting sort; within a row the
-  // samples appear in increasing order), for the adjoint's gather.
-  const int64_t ng = n2 * n2;
-  std::vector<int> rp((size_t)(ng + 1), 0);
   auto wrap = [&](int64_t v) { return (int)((n + v + n2) % n2); };
-  for (int64_t si = 0; si < S; ++si)
-    for (int i1 = 0; i1 < L; ++i1)
-      for (int i0 = 0; i0 < L; ++i0)
-        ++rp[(size_t)(wrap(tb[(size_t)si].y + i1) * n2 + wrap(tb[(size_t)si].x + i0) + 1)];
-  for (int64_t g = 0; g < ng; ++g) rp[(size_t)(g + 1)] += rp[(size_t)g];
-  // grid points with more than kHeavyRow taps, longest first (ties by index)
+  // The samples by 4x4 tile, for the adjoint (counting sort; within a tile the
+  // samples appear in increasing order): a window of 9 taps touches 3 tiles
+  // along each axis, the wrapped first tap's and the next two.  Each list is
+  // padded to a multiple of four with entries whose weights are the zeros at
+  // the rows' ends.
+  const int nt = (int)(n / 2);
+  std::vector<int> tp((size_t)nt * nt + 1, 0);
+  auto tiles3 = [&](int64_t si, auto&& f) {
+    const int wx0 = wrap(tb[(size_t)si].x), wy0 = wrap(tb[(size_t)si].y);
+    for (int jy = 0; jy < 3; ++jy)
+      for (int jx = 0; jx < 3; ++jx)
+        f((wy0 / 4 + jy) % nt * nt + (wx0 / 4 + jx) % nt, 4 * jx - wx0 % 4 + 3, 4 * jy - wy0 % 4 + 3);
+  };
+  for (int64_t si = 0; si < S; ++si) tiles3(si, [&](int t, int, int) { ++tp[(size_t)t + 1]; });
+  std::vector<int> tcnt(tp.begin() + 1, tp.end());
+  for (int t = 0; t < nt * nt; ++t) tp[(size_t)t + 1] = tp[(size_t)t] + (tcnt[(size_t)t] + 3) / 4 * 4;
+  std::vector<int2> te((size_t)std::max(1, tp.back()), make_int2(0, 12 << 8 | 12));
+  {
+    std::vector<int> fill(tp.begin(), tp.end() - 1);
+    for (int64_t si = 0; si < S; ++si)
+      tiles3(si, [&](int t, int ox, int oy) { te[(size_t)fill[(size_t)t]++] = make_int2((int)si, oy << 8 | ox); });
+  }
   std::vector<int> heavy;
-  for (int64_t g = 0; g < ng; ++g)
-    if (rp[(size_t)(g + 1)] - rp[(size_t)g] > kHeavyRow) heavy.push_back((int)g);
+  for (int t = 0; t < nt * nt; ++t)
+    if (tp[(size_t)t + 1] - tp[(size_t)t] > kHeavyTile) heavy.push_back(t);
   std::stable_sort(heavy.begin(), heavy.end(), [&](int x, int y) {
-    return rp[(size_t)x + 1] - rp[(size_t)x] > rp[(size_t)y + 1] - rp[(size_t)y];
+    return tp[(size_t)x + 1] - tp[(size_t)x] > tp[(size_t)y + 1] - tp[(size_t)y];
   });
-  std::vector<int> fill(rp.begin(), rp.end() - 1);
-  std::vector<int2> csw((size_t)(S * L * L));
-  for (int64_t si = 0; si < S; ++si)
-    for (int i1 = 0; i1 < L; ++i1) {
-      const float wy = tw[(size_t)((L + i1) * S + si)];
-      for (int i0 = 0; i0 < L; ++i0) {
-        const int64_t g = wrap(tb[(size_t)si].y + i1) * n2 + wrap(tb[(size_t)si].x + i0);
-        const int k = fill[(size_t)g]++;
-        const float w = wy * tw[(size_t)(i0 * S + si)];
-        int wb;
-        std::memcpy(&wb, &w, sizeof wb);
-        csw[(size_t)k] = make_int2((int)si, wb);
-      }
-    }
   // Tile binning of the samples for the forward gather: tile of the window's
   // first tap (wrapped), sorted by tile (counting sort, samples in increasing
   // order within a tile), cut into work items of at most 256 samples.
@@ -993,6 +1020,7 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
       items.push_back(make_int4(tile % ntx, tile / ntx, b, std::min(256, tcount[(size_t)(tile + 1)] - b)));
   p->nitems = (int)items.size();
   p->nheavy = (int)heavy.size();
+  p->longest = heavy.empty() ? 0 : tp[(size_t)heavy[0] + 1] - tp[(size_t)heavy[0]];
   p->ts = ts;
   // deapodiser phi (tomo.py:19-21, 46-47) with the mask folded in
   std::vector<float> phi((size_t)(n * n));
@@ -1027,8 +1055,8 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
     return r;
   };
   if (e != hipSuccess || (e = up(&p->phi, phi)) != hipSuccess || (e = up(&p->tw2, twid(2 * n))) != hipSuccess ||
-      (e = up(&p->tw1, twid(n))) != hipSuccess || (e = up(&p->tb, tb)) != hipSuccess ||
-      (e = up(&p->tw, tw)) != hipSuccess || (e = up(&p->rp, rp)) != hipSuccess || (e = up(&p->csw, csw)) != hipSuccess ||
+      (e = up(&p->tw1, twid(n))) != hipSuccess || (e = up(&p->wt, wt)) != hipSuccess ||
+      (e = up(&p->tp, tp)) != hipSuccess || (e = up(&p->te, te)) != hipSuccess ||
       (e = up(&p->items, items)) != hipSuccess ||
       (!heavy.empty() && (e = up(&p->heavy, heavy)) != hipSuccess) ||
       (e = up(&p->so, so)) != hipSuccess || (e = up(&p->sf, sf)) != hipSuccess ||
@@ -1045,10 +1073,9 @@ int htamd_tomo_plan_destroy(htamd_tomo_plan* p) {
   (void)hipFree(p->phi);
   (void)hipFree(p->tw2);
   (void)hipFree(p->tw1);
-  (void)hipFree(p->tb);
-  (void)hipFree(p->tw);
-  (void)hipFree(p->rp);
-  (void)hipFree(p->csw);
+  (void)hipFree(p->wt);
+  (void)hipFree(p->tp);
+  (void)hipFree(p->te);
   (void)hipFree(p->items);
   (void)hipFree(p->so);
   (void)hipFree(p->sf);
@@ -1084,19 +1111,19 @@ static int tomo_run(const htamd_tomo_plan* p, bool adjoint, const void* in, int 
   a.ntheta = (int)p->ntheta;
   a.m = p->m;
   a.phi = p->phi;
-  a.tb = p->tb;
-  a.tw = p->tw;
-  a.rp = p->rp;
-  a.csw = p->csw;
+  a.wt = p->wt;
+  a.tp = p->tp;
+  a.te = p->te;
   a.tw2 = p->tw2;
   a.tw1 = p->tw1;
-  a.items = p->m == (kTL - 1) / 2 ? p->items : nullptr;  // the tiled gather is built for 9x9 windows
+  a.items = p->items;
   a.so = p->so;
   a.sf = p->sf;
   a.ts = p->ts;
   a.nitems = p->nitems;
   a.heavy = p->heavy;
   a.nheavy = p->nheavy;
+  a.longest = p->longest;
   a.cxs = (float)(-M_PI * M_PI / p->mu / (4.0 * (double)p->n * (double)p->n));
   a.cys = (float)(M_PI / p->mu);
   a.W = (float2*)ws;

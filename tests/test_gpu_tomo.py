@@ -235,3 +235,24 @@ def test_rec_tomo_matches_oracle(gpu):
     ref8 = np.linalg.norm(o.R(o.rec_tomo(d64, 8)) - d64) ** 2
     print(f"[rec_tomo] objective after 8 iterations: {objs[-1]:.6e} (oracle {ref8:.6e})", flush=True)
     assert abs(objs[-1] - ref8) / ref8 < 1e-2
+
+
+@pytest.mark.parametrize("n,ntheta,nz", [(n, t, z) for n, t in ((10, 7), (50, 200), (64, 96))
+                                         for z in (1, 2, 15, 16, 17, 33, 48, 49, 64, 65, 115)] + [(8, 3, 2561)])
+def test_slab_sizes_at_the_edges_of_the_slice_blocks(gpu, n, ntheta, nz):
+    """Slab sizes around the slice blocks of the gridding products (16, 32, 48
+    and 64 slices, even shares of larger slabs, a last block of one), grids whose tiles do not fill
+    a workgroup's row (n = 10, 50), lists of the central tiles short and long
+    (200 angles: over 1000 samples).  Each slice by itself meets the bar of an
+    81-tap FP32 sum and two FP32 FFTs."""
+    from holotomocupy_amd import Tomo
+    print(f"[case] slab n={n} ntheta={ntheta} nz={nz}", flush=True)
+    rng = np.random.default_rng(n + nz)
+    th = angles(ntheta)
+    g, o = Tomo(n, nz, th, 0), ot.Tomo(n, nz, th, 0)
+    x, d = data(rng, (nz, n, n), False), data(rng, (ntheta, nz, n), False)
+    y, z = g.R(dev(x)).cpu().numpy(), g.RT(dev(d)).cpu().numpy()
+    yo, zo = o.R(x.astype(np.complex128)), o.RT(d.astype(np.complex128))
+    for k in range(nz):
+        assert rel(y[:, k], yo[:, k]) < REL_TOL, k
+        assert rel(z[k], zo[k]) < REL_TOL, k

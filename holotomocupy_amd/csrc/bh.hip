@@ -44,7 +44,7 @@ struct BhArgs {
   float2* part_g = nullptr;          // split angles: [groups <= nang, ndist, nz, n] probe-gradient sums of the
                                      // groups (NULL: not split)
   int64_t maxgroups = 0;             // no more groups than this
-  int kper = 0;                      // angles per workgroup of K1
+  int64_t groups = 1;                // groups of angles of K1
   const float2* twx = nullptr;
   const float2* twy = nullptr;
   const float2* tabx = nullptr;      // [ndist][2][3*(n/2)]
@@ -161,8 +161,8 @@ __device__ __forceinline__ float2 row_sum2(float2 v, float2* red) {
 }
 
 // ---- K1: rows, forward ------------------------------------------------------
-// Workgroup = ROWS row units (j, ty) and kper consecutive angles, over which it
-// loops.  The angles are independent: where the row units alone leave the chip
+// Workgroup = ROWS row units (j, ty) and one of a.groups shares of the angles,
+// over which it loops.  The angles are independent: where the row units alone leave the chip
 // idle (256^2 at 2 distances: 64 workgroups for 256 CUs) the host splits them
 // over more workgroups (kFwdBlocks; 684 -> 57 us for 48 angles there).
 // Four waves per SIMD (at most 128 VGPRs): the staged gather waits on memory
@@ -175,11 +175,11 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(4))
   __shared__ float2 lds[ROWS * fft_buf<N>()];
   const int r = threadIdx.x / T, t0 = threadIdx.x % T;
   const int64_t nunits = (int64_t)a.ndist * a.nz;
-  // each XCD takes whole groups of angles (their object planes stay in its L2)
   const int64_t ublocks = (nunits + ROWS - 1) / ROWS;
-  const int64_t bid = xcd_tile(blockIdx.x, gridDim.x);
-  const int64_t unit = bid % ublocks * ROWS + r;
-  const int64_t b0 = bid / ublocks * a.kper, b1 = min(b0 + a.kper, a.nang);
+  const bool own = a.groups >= kXcdGroups;  // each XCD takes whole groups
+  const int64_t bid = own ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x, q = bid / ublocks;
+  const int64_t unit = (own ? bid - q * ublocks : row_tile(bid - q * ublocks, ublocks, a.ndist)) * ROWS + r;
+  const int64_t b0 = a.nang * q / a.groups, b1 = a.nang * (q + 1) / a.groups;
   const bool valid = unit < nunits;
   const int j = valid ? (int)(unit / a.nz) : 0, ty = valid ? (int)(unit % a.nz) : 0;
   float2* s = lds + r * fft_buf<N>();
@@ -364,12 +364,12 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   __shared__ float2 red[kRowThreads / 64];
   const int r = threadIdx.x / T, t0 = threadIdx.x % T;
   const int64_t nunits = (int64_t)a.ndist * a.nz;
-  // XCD-contiguous row bands.  SPLIT: group after group; workgroups without one
+  // SPLIT: group after group; workgroups without one
   // are the last ones of the launch (dispatched among the others they would
   // leave the same shader engines idle each time)
   const int64_t ublocks = (nunits + ROWS - 1) / ROWS;
   const int64_t q = SPLIT ? blockIdx.x / ublocks : 0;
-  const int64_t unit = xcd_tile(blockIdx.x - q * ublocks, ublocks) * ROWS + r;
+  const int64_t unit = row_tile(blockIdx.x - q * ublocks, ublocks, a.ndist) * ROWS + r;
   const int64_t b0 = SPLIT ? group_start(a.pidx, a.nang, q) : 0;
   if (b0 >= a.nang) return;  // the whole workgroup
   const int64_t b1 = SPLIT ? min(b0 + kAdjGroup, a.nang) : a.nang;
@@ -665,23 +665,6 @@ struct BhLayout {
   int64_t c = 0, T = 0, dpsi = 0, part_r = 0, part_obj = 0, part_g = 0, total = 0;
 };
 
-// Workgroups of row units (j, ty) of one angle in the row passes.
-static int64_t row_blocks(int64_t n, int64_t nz, int64_t ndist) {
-  const int64_t rows = n >= 2048 ? 1 : kRowThreads / (n / 8);
-  return (ndist * nz + rows - 1) / rows;
-}
-
-// K3 splits the angles into groups (see there) when one angle's row units are
-// fewer than this (two or three workgroups of it fit a CU, 512 to 768 the chip).
-// 256^2, 2 distances, 48 angles (64 workgroups of row units): 815 -> 149 us and
-// 5 us for bh_prb_final_k; 1024^2 at 3 distances and 16 angles (1536): the whole
-// gradient 1697 against 1697 us; at 2048 and more the extra field of group sums
-// would only cost.
-constexpr int64_t kAdjSplitBelow = 2048;
-static bool adj_split(int64_t n, int64_t nz, int64_t ndist) { return row_blocks(n, nz, ndist) < kAdjSplitBelow; }
-// K1 splits the angles over workgroups until there are about this many.
-constexpr int64_t kFwdBlocks = 4096;
-
 // Column pass of the fused gradient: 16 elements per thread at N = 2048 (two
 // columns per 256-thread workgroup), else 8.
 template <int N>
@@ -724,6 +707,47 @@ static int cols_per_tile(int64_t nz, int64_t n) {
   }
 }
 
+// LDS of one workgroup: the statically sized buffers plus the staged object
+// rows (one row of npsi values per detector row, two in the adjoint pass);
+// rows are staged when the staged part fits 64 KiB and the total the 160 KiB
+// of a CU.
+constexpr int64_t kRowDynBudget = 65536;
+constexpr int64_t kRowLdsBudget = 160 * 1024;
+
+// Row units per workgroup and LDS of a row pass.
+struct RowShape {
+  int64_t blocks = 0, dyn = 0, lds = 0;
+  bool staged = false;
+};
+static RowShape row_shape(int64_t n, int64_t nz, int64_t ndist, int64_t npsi, int64_t osz, bool adjoint) {
+  RowShape r;
+  const int64_t rows = kRowThreads / (n / 8), fbuf = n + n / 16;
+  const int64_t stat = rows * (fbuf + (adjoint ? n : 0)) * 8 + 64;
+  r.dyn = rows * npsi * osz * (adjoint ? 2 : 1);
+  r.staged = r.dyn <= kRowDynBudget && stat + r.dyn <= kRowLdsBudget;
+  if (!r.staged) r.dyn = 0;
+  r.lds = stat + r.dyn;
+  r.blocks = (ndist * nz + rows - 1) / rows;
+  return r;
+}
+
+// K3 splits the angles into groups (see there) where one angle's row units are
+// fewer than kAdjSplitBelow workgroups and do not fill rounds of the chip
+// (registers admit three workgroups per CU, their LDS often two).  256^2, 2
+// distances, 48 angles (64 workgroups): 815 -> 149 us and 5 us for
+// bh_prb_final_k; the whole gradient at 1024^2, 2 distances, 32 angles: with
+// 512^2 objects (1024 workgroups in rounds of 768) 2500 -> 2320 us, with 1024^2
+// ones (two rounds of 512, not split) split 1979 -> 2002 us.
+constexpr int64_t kAdjSplitBelow = 2048;
+static bool adj_split(int64_t n, int64_t nz, int64_t ndist, int64_t npsi, int64_t osz) {
+  const RowShape r = row_shape(n, nz, ndist, npsi, osz, true);
+  return r.blocks < kAdjSplitBelow && !whole_rounds(r.blocks, 3, r.lds, 2);
+}
+// K1 splits the angles over workgroups until there are about this many, unless
+// one angle's row units are one whole round (1024^2, 2 distances, 16 angles:
+// split 1979 -> 2002 us).
+constexpr int64_t kFwdBlocks = 4096;
+
 static BhLayout bh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* sp, int64_t nang) {
   BhLayout L;
   const int64_t osz = sp->is_complex ? 8 : 4;
@@ -742,17 +766,10 @@ static BhLayout bh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* sp,
   L.part_obj = off;
   off += align256(ntiles * 8);
   L.part_g = off;
-  if (adj_split(pp->n, pp->nz, pp->ndist)) off += align256(nang * pp->ndist * field * 8);
+  if (nang > kAdjGroup && adj_split(pp->n, pp->nz, pp->ndist, sp->npsi, osz)) off += align256(nang * pp->ndist * field * 8);
   L.total = off;
   return L;
 }
-
-// LDS of one workgroup: the statically sized buffers plus the staged object
-// rows (one row of npsi values per detector row, two in the adjoint pass);
-// rows are staged when the staged part fits 64 KiB and the total the 160 KiB
-// of a CU.
-constexpr int64_t kRowDynBudget = 65536;
-constexpr int64_t kRowLdsBudget = 160 * 1024;
 
 // Row-pass elements per thread (one row per 256 threads at N = 2048; 16
 // elements with radix-16 stages measured slower: fewer waves per CU).
@@ -764,16 +781,12 @@ constexpr int bh_row_e() {
 template <int N, typename TO>
 static hipError_t launch_rows(bool adjoint, BhArgs a, hipStream_t st) {
   constexpr int E = bh_row_e<N>();
-  constexpr int ROWS = kRowThreads / (N / E);
   const int64_t units = (int64_t)a.ndist * a.nz;
-  const int64_t ublocks = (units + ROWS - 1) / ROWS;
-  const int64_t groups = std::min(a.nang, (kFwdBlocks + ublocks - 1) / ublocks);
-  a.kper = (int)((a.nang + groups - 1) / groups);
-  const bool split = a.part_g != nullptr;
-  const int64_t grid = ublocks * (!adjoint ? (a.nang + a.kper - 1) / a.kper : split ? a.maxgroups : 1);
-  const int64_t stat = (int64_t)ROWS * (fft_buf<N>() + (adjoint ? N : 0)) * 8 + 64;
-  const int64_t dyn = (int64_t)ROWS * a.npsi * (int64_t)sizeof(TO) * (adjoint ? 2 : 1);
-  const bool staged = dyn <= kRowDynBudget && stat + dyn <= kRowLdsBudget;
+  const RowShape rs = row_shape(N, a.nz, a.ndist, a.npsi, sizeof(TO), adjoint);
+  const int64_t dyn = rs.dyn;
+  const bool staged = rs.staged, split = a.part_g != nullptr;
+  a.groups = whole_rounds(rs.blocks, 4, rs.lds, 1) ? 1 : std::min(a.nang, (kFwdBlocks + rs.blocks - 1) / rs.blocks);
+  const int64_t grid = rs.blocks * (!adjoint ? a.groups : split ? a.maxgroups : 1);
   if (adjoint) {
     if (staged && split)
       hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, true, true>), dim3((unsigned)grid), dim3(kRowThreads),
@@ -999,7 +1012,7 @@ static int bh_gradient_impl(const htamd_bh_plan* p, int64_t nangles, const void*
   a.accumulate_prb = accumulate_prb;
   a.part_r = (float2*)(ws + L.part_r);
   a.part_obj = (double*)(ws + L.part_obj);
-  if (nangles > kAdjGroup && adj_split(a.n, a.nz, a.ndist)) {  // up to one group: the same sum either way
+  if (nangles > kAdjGroup && adj_split(a.n, a.nz, a.ndist, a.npsi, p->shift->is_complex ? 8 : 4)) {  // up to one group: the same sum either way
     a.part_g = (float2*)(ws + L.part_g);
     // a run ends at most one group early; nprobes is not known without the table
     const int64_t full = (nangles + kAdjGroup - 1) / kAdjGroup;

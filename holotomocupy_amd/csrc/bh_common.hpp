@@ -46,6 +46,34 @@ struct StageEvents {
   }
 };
 
+// Workgroup -> row units of the row passes.  Contiguous bands put the XCDs
+// ndist nz n bytes apart, which with one to three distances costs up to 9%
+// against chunks of 16 workgroups in turn (gradient at 2048^2, 16 angles: 1
+// distance 2706 -> 2462 us, 2 distances 8 angles 2493 -> 2299 us; 1024^2, 2
+// distances 2334 -> 2160 us).  From four distances on the bands are distances
+// whose rows sample the same object rows at the same time, and are better (4
+// distances: 8264 against 8327 us; bilinear pair at 1024^2 4422 against 4515).
+__device__ __forceinline__ int64_t row_tile(int64_t bid, int64_t nblocks, int ndist) {
+  return ndist >= 4 ? xcd_tile(bid, nblocks) : xcd_chunks<16>(bid, nblocks);
+}
+
+// With at least this many groups of angles each XCD takes whole groups instead
+// (gradient at 256^2, 2 distances, 48 angles: 417 -> 407 us; equal form at
+// 256^2, 3 distances, 64 angles 637 -> 618 us).
+constexpr int kXcdGroups = 8;
+
+constexpr int64_t kNumCu = 256, kCuLds = 160 * 1024;
+
+// Whether `blocks` workgroups, of which a CU holds per_cu (at most waves_cu
+// by their registers, and what their LDS leaves room for), run in whole
+// rounds of the chip, or nearly so, and in at most `most` of them.
+inline bool whole_rounds(int64_t blocks, int64_t waves_cu, int64_t lds, int64_t most) {
+  const int64_t by_lds = lds > 0 ? kCuLds / lds : waves_cu;
+  const int64_t per_round = kNumCu * (by_lds < 1 ? 1 : by_lds < waves_cu ? by_lds : waves_cu);
+  const int64_t rounds = (blocks + per_round - 1) / per_round;
+  return rounds <= most && 10 * blocks >= 9 * rounds * per_round;
+}
+
 inline int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 }  // namespace htamd

@@ -80,21 +80,21 @@ struct HessShape {
 // place.  Nothing is held across transforms, so no per-pixel array is kept
 // (the fused form held four or five complex values per pixel across its NF
 // transforms, in scratch).  A workgroup = rpb row units (j, ty) of T = N/E
-// threads and kper consecutive angles, over which it loops.  rpb <=
-// kRowThreads / T, chosen so the staged rows fit the dynamic LDS.
+// threads and one of `groups` shares of the angles, over which it loops.  rpb
+// <= kRowThreads / T, chosen so the staged rows fit the dynamic LDS.
 template <int N, int E, typename TO, int MODE>
-__global__ __launch_bounds__(kRowThreads) void bhh_chain_k(BhhArgs a, int rpb, int kper) {
+__global__ __launch_bounds__(kRowThreads) void bhh_chain_k(BhhArgs a, int rpb, int groups) {
   using HS = HessShape<MODE>;
   constexpr bool SAME = HS::SAME, PAIR = HS::PAIR;
   constexpr int T = N / E;
   constexpr int NR = HS::NR;
   const int r = threadIdx.x / T, t0 = threadIdx.x % T;
   const int64_t nunits = (int64_t)a.ndist * a.nz;
-  // each XCD takes whole groups of angles (their object planes stay in its L2)
   const int64_t ublocks = (nunits + rpb - 1) / rpb;
-  const int64_t bid = xcd_tile(blockIdx.x, gridDim.x);
-  const int64_t unit = bid % ublocks * rpb + r;
-  const int64_t b0 = bid / ublocks * kper, b1 = min(b0 + kper, a.nang);
+  const bool own = groups >= kXcdGroups;  // each XCD takes whole groups
+  const int64_t bid = own ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x, q = bid / ublocks;
+  const int64_t unit = (own ? bid - q * ublocks : row_tile(bid - q * ublocks, ublocks, a.ndist)) * rpb + r;
+  const int64_t b0 = a.nang * q / groups, b1 = a.nang * (q + 1) / groups;
   const bool valid = unit < nunits;
   const int j = valid ? (int)(unit / a.nz) : 0, ty = valid ? (int)(unit % a.nz) : 0;
   const int64_t plane = (int64_t)a.nzpsi * a.npsi;
@@ -518,8 +518,10 @@ static BhhLayout bhh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* s
 // Row pass: 8 elements per thread as the gradient's row passes; the staged
 // rows of a workgroup stay within 64 KiB of dynamic LDS.
 constexpr int64_t kHessDynBudget = 65536;
-// The chain kernel's angles are independent: they are split over workgroups until there are about this many
-// (pair form at 256^2, 4 distances, 32 angles: 781 -> 541 us in all; 1024^2, 16 angles, from 2048: 4539 -> 4351 us).
+// The chain kernel's angles are independent: they are split over workgroups until there are about this many, unless
+// one angle's row units are one whole round.  Pair form at 256^2, 4 distances, 32 angles: 781 -> 541 us in all;
+// 1024^2, 16 angles, 512^2 objects (2048 workgroups): 4533 -> 4427 us; equal form at 1024^2, 1 distance, 22 angles,
+// 1024^2 objects (512, one round): split 1600 -> 1623 us.
 constexpr int64_t kHessBlocks = 4096;
 
 template <int N, typename TO, int MODE>
@@ -531,11 +533,12 @@ static hipError_t hess_rows_m(const BhhArgs& a, hipStream_t st) {
   while (rpb > 1 && rpb * per_row > kHessDynBudget) rpb >>= 1;
   if (rpb * per_row > kHessDynBudget) return hipErrorInvalidConfiguration;
   const int64_t ublocks = ((int64_t)a.ndist * a.nz + rpb - 1) / rpb;
-  const int64_t groups = std::min(a.nang, (kHessBlocks + ublocks - 1) / ublocks);
-  const int64_t kper = (a.nang + groups - 1) / groups;
-  const int64_t grid = ublocks * ((a.nang + kper - 1) / kper);
+  const int64_t groups = whole_rounds(ublocks, 4, rpb * per_row, 1)
+                             ? 1
+                             : std::min(a.nang, (kHessBlocks + ublocks - 1) / ublocks);
+  const int64_t grid = ublocks * groups;
   hipLaunchKernelGGL((bhh_chain_k<N, E, TO, MODE>), dim3((unsigned)grid), dim3(rpb * T), (size_t)(rpb * per_row),
-                     st, a, rpb, (int)kper);
+                     st, a, rpb, (int)groups);
   return hipGetLastError();
 }
 

@@ -52,4 +52,14 @@ __device__ __forceinline__ int64_t xcd_tile(int64_t bid, int64_t nblocks) {
   return xcd * per + (xcd < rem ? xcd : rem) + local;
 }
 
+// The same in chunks: XCD x gets tiles [x CH, (x + 1) CH), [(8 + x) CH, ...) and
+// so on, so the tiles in flight on the eight XCDs are one contiguous range.
+template <int CH>
+__device__ __forceinline__ int64_t xcd_chunks(int64_t bid, int64_t nblocks) {
+  constexpr int64_t span = (int64_t)kNumXcd * CH;
+  if (bid >= nblocks / span * span) return bid;  // the rest in order
+  const int64_t xcd = bid % kNumXcd, local = bid / kNumXcd;
+  return (local / CH * kNumXcd + xcd) * CH + local % CH;
+}
+
 }  // namespace htamd

@@ -1,7 +1,7 @@
 // USFFT Radon transform R / RT for gfx950 (src/holotomocupy/tomo.py:12-116,
 // gridding kernel src/holotomocupy/cuda_kernels.py:3-76).
 //
-//   R(obj)  = c1d IFFT1(c1d gather(c2d FFT2(c2d embed(obj phi))) / n) / 4
+//   R(obj)  = c1d IFFT1(c1d gather(c2d FFT2(c2d embed(obj phi))) / n) / 4   (1/n applied with the 1/4, rounded once)
 //   RT(d)   = crop(c2d IFFT2(c2d scatter(c1d FFT1(c1d d)))) phi
 //
 // c1d[k] = (-1)^(k+1), c2d[i,j] = (-1)^(i+j) on the 2n x 2n grid.  The 2-D
@@ -9,11 +9,11 @@
 // non-zero rows of the embedded slice are transformed along x), with the sign
 // modulations, zero-embedding, cropping and deapodisation folded into the
 // loads and stores.  The 9x9 Gaussian gridding taps of every polar sample are
-// built once per plan in FP64 (stored FP32): the forward gathers them through
-// LDS tiles of the grid; the adjoint sorts the samples by 4x4 tile of the grid
-// and forms each tile as a matrix product over its samples, from a
-// slice-contiguous copy of the transformed sinogram -- the reference's atomic
-// scatter in a fixed summation order.
+// built once per plan in FP64 (stored FP32).  Between the grid and the line
+// spectra (slices fastest) both directions are matrix products over all
+// slices: the forward over groups of samples whose windows share a patch of the
+// grid, the adjoint over 4x4 tiles of the grid and the samples that touch them
+// -- the reference's atomic scatter in a fixed summation order.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -27,6 +27,11 @@
 #include "htamd_internal.hpp"
 
 namespace htamd {
+
+constexpr int kWRow = 16;  // a sample's weights along an axis: 3 zeros, 9 taps, 4 zeros
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(8)));  // an odd slice count leaves rows 8-byte aligned
 
 struct TomoArgs {
   int n = 0, nz = 0, ntheta = 0, m = 0;
@@ -42,19 +47,19 @@ struct TomoArgs {
   // index in the sample's x weights of the tile's first column (oy of its row)
   const int* tp = nullptr;
   const int2* te = nullptr;
-  // the samples binned by grid tile for the forward gather: work item i covers
-  // samples [it.z, it.z + it.w) of the sorted list, all in tile (it.x, it.y);
-  // per sorted sample: (local tap origin oy << 16 | ox, sample index) and the
-  // fractional parts (frac(2n x0), frac(2n y0)) that give its weights
+  // the samples for the forward gather: groups of up to 16 whose first taps lie
+  // in one cell of 4 rows x 8 columns, ge[16 g + i] = (sample or -1, oy << 8 |
+  // ox) with (oy, ox) the first tap's place in the cell; gc[g] = the cell's
+  // place in its region (row << 8 | column); work item = (column, row of the
+  // kRG x kRG region, first group, groups)
   const int4* items = nullptr;
-  const int2* so = nullptr;
-  const float2* sf = nullptr;
-  int ts = 0;                      // tile edge on the 2n grid
+  const int2* ge = nullptr;
+  const int* gc = nullptr;
   int nitems = 0;
-  float cxs = 0.f, cys = 0.f;      // weights exp(cxs (i - m - f)^2), cys exp(...)
+  int sparse = 0;                  // the groups are of regions, one to a work item
   float2* W = nullptr;             // [nz, n, 2n]
   float2* G = nullptr;             // [nz, 2n, 2n]
-  float2* Sh = nullptr;            // [ntheta n, nz] transformed sinogram (RT)
+  float2* Sh = nullptr;            // [ntheta n, nz] line spectra, slices fastest
   const int* heavy = nullptr;      // tiles with more than kHeavyTile entries, longest first
   int nheavy = 0;
   int longest = 0;                 // entries of the longest list
@@ -141,139 +146,229 @@ __global__ __launch_bounds__(C*(N2 / E)) void tomo_cols_fwd_k(TomoArgs a) {
   }
 }
 
-// ---- forward pass C, tiled: gather through LDS tiles of the grid ------------
-// The polar samples are binned by the grid tile holding the first tap of
-// their 9x9 window (plan time).  A workgroup takes one work item (up to 256
-// samples of one tile) for kTZ slices: it stages the tile plus the window
-// margin, wrapped on the 2n grid, into LDS for each slice, and each thread
-// gathers its sample's taps from LDS.  The weights come from the sample's
-// fractional grid offset, exp(-pi^2/mu ((i - m - f)/(2n))^2) evaluated in
-// FP32 (the FP64-built offset keeps the argument accurate).  The sums run in
-// the order of the untiled gather (rows outer, columns inner).  Output: the
-// line spectra Sh[(theta nz + z) n + t], scaled by c1d / n.
-constexpr int kTS = 32, kTL = 9, kTP = kTS + kTL - 1, kTZ = 4;
-__global__ __launch_bounds__(256) void tomo_tile_gather_k(TomoArgs a) {
-  static_assert(kTZ == 4, "a staged point's slices are two float4");
-  // slice-minor: point (r, c) holds its kTZ slices at tile[(r kTP + c) kTZ + q],
-  // so a tap's four slices are two 16-byte LDS reads
-  __shared__ float4 tile4[kTP * kTP * kTZ / 2];
-  float2* tile = reinterpret_cast<float2*>(tile4);
-  const int4 it = a.items[blockIdx.x];
-  const int z0 = blockIdx.y * kTZ;
-  const int n2 = 2 * a.n, P = a.ts + kTL - 1;
+// ---- forward pass C: the grid at the samples ---------------------------------
+// Sh[s][z] = c1d sum over the 9x9 window of sample s of wy wx G[z][g], as the
+// adjoint (see tomo_grid_k) in FP32 matrix products.  Up to 16 samples whose
+// windows start in one cell of 4x8 points have their windows inside 12 rows of
+// 16 points: a row is a product of 16 slices x 16 points with the 16 x 16
+// matrix of x weights, and its result is added with the lane's sample's y
+// weight, as the sum per sample would.
+// 81 of the patch's 192 points count for a sample, and far from the centre a
+// cell holds about 8 samples at 256^2, 384 angles: 4x4 cells take a third more
+// products, 8x8 cells as many more at that density (fewer at sparser ones).
+// A workgroup stages a region of kRG x kRG first taps with the margin of the
+// windows, wrapped on the 2n grid, for 16 slices (slices fastest, a point's
+// row padded to 17: the lanes of a read are 16 slices of 4 neighbouring
+// points, the lanes of a staging write 12 pairs of points of one slice), and
+// its wavefronts take the groups in turn.
+// Each sample's two weight rows are read once per group; lane l holds sample
+// l % 16 and the points 4 j + l / 16 of a row.
+// Few angles leave a cell one or two samples: then a group is 16 samples of a
+// region (SPARSE), a workgroup takes one group, and its wavefronts share the
+// rows of the region's patch.  The plan takes the form of fewer steps (R at 8
+// slices of 512^2, 64 angles: 111 us with cells, 92 with regions; 100 slices of
+// 256^2, 100 angles: 272 and 316).
+// 256 slices of 256^2, 384 angles: 974 us with a thread per sample and four
+// slices -> 450 us (the products are 177 us).
+constexpr int kTL = 9;                        // taps along an axis
+constexpr int kRG = 16, kRP = kRG + kTL - 1;  // region and its staged edge
+constexpr int kRZ = 16, kRZP = kRZ + 1;       // slices, and the pitch of a staged point
+constexpr int kCellY = 4, kCellX = 8;
+constexpr int kItemGroups = 16;               // groups of a work item
+constexpr int kGatherWaves = 8;
+constexpr int kStageSteps = 96;               // a region's staging, in steps of products (see the plan)
+
+// The patch of points a group's windows lie in: that of one cell, or (SPARSE)
+// of the whole region.
+template <bool SPARSE>
+struct GatherShape {
+  static constexpr int NY = SPARSE ? kRP : kCellY + kTL - 1;                 // rows
+  static constexpr int NX = (SPARSE ? kRP : kCellX + kTL - 1) / 4;           // steps of a row
+  static constexpr int NR = SPARSE ? kRP / kGatherWaves : NY;                // rows of a wavefront
+};
+
+template <bool SPARSE>
+__global__ __launch_bounds__(64 * kGatherWaves) __attribute__((amdgpu_waves_per_eu(4))) void tomo_gather_k(
+    TomoArgs a, int zper) {
+  using S = GatherShape<SPARSE>;
+  __shared__ float2 tile[kRP * kRP * kRZP];
+  const int4 it = a.items[xcd_tile(blockIdx.x, gridDim.x)];
+  const int z0 = blockIdx.y * zper, nzb = min(zper, a.nz - z0);
+  const int n2 = 2 * a.n;
   const int64_t plane = (int64_t)n2 * n2;
-  const int gy0 = it.y * a.ts, gx0 = it.x * a.ts;
-  // staged element (q, r, c) by the compile-time pitch kTP (the divisions are
-  // multiply-shifts), slice fastest so consecutive threads fill consecutive
-  // LDS slots; the wrap onto the 2n grid is one conditional subtraction: the
-  // tile origin is a multiple of ts below 2n and r, c < ts + 8, which keeps
-  // origin + r below 4n for every even n >= 8
-  for (int idx = threadIdx.x; idx < kTZ * kTP * kTP; idx += 256) {
-    const int pt = idx / kTZ, q = idx - pt * kTZ;
-    const int r = pt / kTP, c = pt - r * kTP;
-    if (r >= P || c >= P) continue;  // tiles narrower than kTS (2n < kTS)
-    const int z = z0 + q;
-    int gr = gy0 + r, gc = gx0 + c;
+  const int gy0 = it.y * kRG, gx0 = it.x * kRG;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int q = lane & 15, kk = lane >> 4;
+  constexpr int PP = kRP / 2;  // pairs of points of a row (2n is even: the wrap splits none)
+  constexpr int NT = 64 * kGatherWaves, NP = kRZ * kRP * PP;
+  static_assert(NP % NT == 0, "every thread stages the same number of pairs");
+  f32x4 v[NP / NT];
+#pragma unroll
+  for (int k = 0; k < NP / NT; ++k) {
+    const int idx = threadIdx.x + k * NT, zr = idx / PP, x = (idx - zr * PP) * 2;
+    const int z = zr / kRP, r = zr - z * kRP;
+    int gr = gy0 + r, gx = gx0 + x;
     gr -= gr >= n2 ? n2 : 0;
-    gc -= gc >= n2 ? n2 : 0;
-    tile[idx] = z < a.nz ? a.G[z * plane + (int64_t)gr * n2 + gc] : make_float2(0.f, 0.f);
+    gx -= gx >= n2 ? n2 : 0;
+    v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (z < nzb) v[k] = *reinterpret_cast<const f32x4u*>(a.G + (z0 + z) * plane + (int64_t)gr * n2 + gx);
+  }
+#pragma unroll
+  for (int k = 0; k < NP / NT; ++k) {
+    const int idx = threadIdx.x + k * NT, zr = idx / PP, x = (idx - zr * PP) * 2;
+    const int z = zr / kRP, r = zr - z * kRP;
+    float2* t = tile + (r * kRP + x) * kRZP + z;
+    t[0] = make_float2(v[k].x, v[k].y);
+    t[kRZP] = make_float2(v[k].z, v[k].w);
   }
   __syncthreads();
-  if ((int)threadIdx.x >= it.w) return;
-  const int k = it.z + threadIdx.x;
-  const int2 so = a.so[k];
-  const float2 f = a.sf[k];
-  const int ox = so.x & 0xffff, oy = so.x >> 16, si = so.y;
-  float wx[kTL];
+  // SPARSE: one group, whose rows the wavefronts share (wv, wv + 8, wv + 16)
+  for (int g = SPARSE ? it.z : it.z + wv; g < it.z + it.w; g += SPARSE ? 1 : kGatherWaves) {
+    const int2 en = a.ge[16 * g + q];
+    const int cell = a.gc[g], s = en.x, ox = en.y & 0xff, oy = en.y >> 8;
+    const float* w = a.wt + (int64_t)max(s, 0) * (2 * kWRow);
+    float wx[S::NX], wy[S::NR];
 #pragma unroll
-  for (int i = 0; i < kTL; ++i) {
-    const float dx = (float)(i - a.m) - f.x;
-    wx[i] = expf(a.cxs * dx * dx);
-  }
-  const int th = si / a.n, t = si % a.n;
-  const float sc = -sgnf(t) / (float)a.n;
-  const float4* tq = tile4 + (oy * kTP + ox) * 2;
-  float2 acc[kTZ];
-#pragma unroll
-  for (int q = 0; q < kTZ; ++q) acc[q] = make_float2(0.f, 0.f);
-#pragma unroll 1
-  for (int i1 = 0; i1 < kTL; ++i1) {  // one tap row at a time (registers)
-    const float dy = (float)(i1 - a.m) - f.y;
-    const float wy = a.cys * expf(a.cxs * dy * dy);
-    float2 racc[kTZ];
-#pragma unroll
-    for (int q = 0; q < kTZ; ++q) racc[q] = make_float2(0.f, 0.f);
-#pragma unroll
-    for (int i0 = 0; i0 < kTL; ++i0) {
-      const float4 v01 = tq[(i1 * kTP + i0) * 2], v23 = tq[(i1 * kTP + i0) * 2 + 1];
-      racc[0] = vfma(wx[i0], make_float2(v01.x, v01.y), racc[0]);
-      racc[1] = vfma(wx[i0], make_float2(v01.z, v01.w), racc[1]);
-      racc[2] = vfma(wx[i0], make_float2(v23.x, v23.y), racc[2]);
-      racc[3] = vfma(wx[i0], make_float2(v23.z, v23.w), racc[3]);
+    for (int j = 0; j < S::NX; ++j) {
+      const int i = 4 * j + kk - ox;  // tap
+      wx[j] = s >= 0 && i >= 0 && i < kTL ? w[3 + i] : 0.f;
     }
 #pragma unroll
-    for (int q = 0; q < kTZ; ++q) acc[q] = vfma(wy, racc[q], acc[q]);
-  }
+    for (int r = 0; r < S::NR; ++r) {
+      const int i = (SPARSE ? wv + r * kGatherWaves : r) - oy;
+      wy[r] = !SPARSE || (i >= 0 && i < kTL) ? w[kWRow + 3 + i] : 0.f;
+    }
+    const float2* base = tile + (((cell >> 8) * kCellY * kRP) + (cell & 0xff) * kCellX + kk) * kRZP + q;
+    if constexpr (SPARSE) base += wv * kRP * kRZP;
+    f32x4 re{0.f, 0.f, 0.f, 0.f}, im{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int q = 0; q < kTZ; ++q)
-    if (z0 + q < a.nz) a.Sh[((int64_t)th * a.nz + z0 + q) * a.n + t] = cscale(acc[q], sc);
+    for (int r = 0; r < S::NR; ++r) {
+      f32x4 ar{0.f, 0.f, 0.f, 0.f}, ai{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < S::NX; ++j) {
+        const float2 b = base[((SPARSE ? r * kGatherWaves : r) * kRP + 4 * j) * kRZP];
+        ar = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, wx[j], ar, 0, 0, 0);
+        ai = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, wx[j], ai, 0, 0, 0);
+      }
+      re += wy[r] * ar;
+      im += wy[r] * ai;
+    }
+    // rows 4 (l / 16) + i are slices, columns q samples; c1d[t] = -(-1)^t, and t
+    // has the parity of s (n is even)
+    auto store = [&](int i, float2 o) {
+      const int z = 4 * kk + i;
+      if (s >= 0 && z < nzb) a.Sh[(int64_t)s * a.nz + z0 + z] = (s & 1) ? o : make_float2(-o.x, -o.y);
+    };
+    if constexpr (SPARSE) {
+      __syncthreads();  // every wavefront has read the tile
+      f32x4* part = reinterpret_cast<f32x4*>(tile);
+      part[(2 * wv) * 64 + lane] = re;
+      part[(2 * wv + 1) * 64 + lane] = im;
+      __syncthreads();
+      if (wv >= 4) return;
+      const float* p = reinterpret_cast<const float*>(tile) + 4 * lane + wv;
+      float2 o = make_float2(0.f, 0.f);
+#pragma unroll
+      for (int k = 0; k < kGatherWaves; ++k) o = cadd(o, make_float2(p[2 * k * 256], p[(2 * k + 1) * 256]));
+      store(wv, o);
+      return;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) store(i, make_float2(re[i], im[i]));
+    }
+  }
 }
 
+static hipError_t launch_gather(const TomoArgs& a, hipStream_t st) {
+  const int zblocks = (a.nz + kRZ - 1) / kRZ, zper = (a.nz + zblocks - 1) / zblocks;
+  const dim3 grid((unsigned)a.nitems, (unsigned)zblocks);
+  if (a.sparse)
+    hipLaunchKernelGGL((tomo_gather_k<true>), grid, dim3(64 * kGatherWaves), 0, st, a, zper);
+  else
+    hipLaunchKernelGGL((tomo_gather_k<false>), grid, dim3(64 * kGatherWaves), 0, st, a, zper);
+  return hipGetLastError();
+}
+
+// Line passes: a workgroup takes C consecutive lines theta nz + z, which
+// mostly are C slices of one angle, so that the slices-fastest spectra are read
+// and written C x 8 bytes at a time (the lanes of a tile access run over the
+// lines), the sinogram along the lines.  C = 16 where 1024 threads and 70 KiB
+// of LDS hold it, 4 below kLineFew lines (one slice of 512^2, 16 angles: 8.5 us
+// with one workgroup of 16 lines).
+template <int N>
+constexpr int line_c() {
+  return N <= 512 ? 16 : 8;
+}
+constexpr int64_t kLineFew = 2048;
+
+// index of (line, t) in the spectra; lines past the end repeat the last
+struct LineIdx {
+  int64_t base;
+  int nz;
+  __device__ __forceinline__ LineIdx(const TomoArgs& a, int64_t line) : nz(a.nz) {
+    const int64_t last = (int64_t)a.ntheta * a.nz - 1;
+    line = line < last ? line : last;
+    const int64_t th = line / a.nz;
+    base = th * a.n * a.nz + (line - th * a.nz);
+  }
+  __device__ __forceinline__ int64_t at(int t) const { return base + (int64_t)t * nz; }
+};
+
 // ---- forward pass D: line IFFT of the gathered spectra ----------------------
-template <int N, int E, typename TO>
-__global__ __launch_bounds__(256) void tomo_line_ifft_k(TomoArgs a, TO* __restrict__ out) {
-  constexpr int T = N / E, ROWS = 256 / T;
-  __shared__ float2 lds[ROWS * fft_buf<N>()];
-  const int r = threadIdx.x / T, t = threadIdx.x % T;
-  const int64_t line = (int64_t)blockIdx.x * ROWS + r;  // theta nz + z
-  const bool valid = line < (int64_t)a.ntheta * a.nz;
-  float2* s = lds + r * fft_buf<N>();
+template <int N, int E, int C, typename TO>
+__global__ __launch_bounds__(C*(N / E)) void tomo_line_ifft_k(TomoArgs a, TO* __restrict__ out) {
+  constexpr int T = N / E, LS = col_stride<N, C>();
+  __shared__ float2 lds[C * LS];
+  const int cc = threadIdx.x / T, t = threadIdx.x % T;
+  const int64_t l0 = (int64_t)blockIdx.x * C;
   FftTw<N, E> twr;
   fft_load_twiddles<N, E>(twr, t, a.tw1);
-  const float2* src = a.Sh + (valid ? line : 0) * N;
+  {
+    const int c = threadIdx.x % C, p0 = threadIdx.x / C;
+    const LineIdx li(a, l0 + c);
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int tt = t + e * T;
-    s[fpad(tt)] = src[tt];
+    for (int e = 0; e < E; ++e) lds[c * LS + fpad(p0 + e * T)] = a.Sh[li.at(p0 + e * T)];
   }
   __syncthreads();
+  float2* s = lds + cc * LS;
   fft_lds<N, E, true>(s, t, twr);
-  if (valid) {
-    TO* dst = out + line * N;
+  if (l0 + cc < (int64_t)a.ntheta * a.nz) {
+    TO* dst = out + (l0 + cc) * N;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int tt = t + e * T;
-      st_c<TO>(dst, tt, cscale(s[fpad(tt)], -sgnf(tt) / (4.0f * N)));
+      st_c<TO>(dst, tt, cscale(s[fpad(tt)], -sgnf(tt) * (float)(0.25 / ((double)N * N))));
     }
   }
 }
 
-// ---- adjoint pass C': line FFT into the z-contiguous sinogram ---------------
-template <int N, int E, typename TI>
-__global__ __launch_bounds__(256) void tomo_linefft_k(TomoArgs a, const TI* __restrict__ data) {
-  constexpr int T = N / E, ROWS = 256 / T;
-  __shared__ float2 lds[ROWS * fft_buf<N>()];
-  const int r = threadIdx.x / T, t = threadIdx.x % T;
-  const int64_t line = (int64_t)blockIdx.x * ROWS + r;  // (theta, z), z fastest
-  const bool valid = line < (int64_t)a.ntheta * a.nz;
-  const int th = valid ? (int)(line / a.nz) : 0;
-  const int z = valid ? (int)(line % a.nz) : 0;
-  float2* s = lds + r * fft_buf<N>();
+// ---- adjoint pass C': line FFT into the slices-fastest spectra --------------
+template <int N, int E, int C, typename TI>
+__global__ __launch_bounds__(C*(N / E)) void tomo_linefft_k(TomoArgs a, const TI* __restrict__ data) {
+  constexpr int T = N / E, LS = col_stride<N, C>();
+  __shared__ float2 lds[C * LS];
+  const int cc = threadIdx.x / T, t = threadIdx.x % T;
+  const int64_t l0 = (int64_t)blockIdx.x * C, lines = (int64_t)a.ntheta * a.nz;
+  const bool valid = l0 + cc < lines;
+  float2* s = lds + cc * LS;
   FftTw<N, E> twr;
   fft_load_twiddles<N, E>(twr, t, a.tw1);
-  const TI* src = data + ((int64_t)th * a.nz + z) * N;
+  const TI* src = data + (valid ? l0 + cc : 0) * N;
+#pragma unroll
   for (int e = 0; e < E; ++e) {
     const int tt = t + e * T;
     s[fpad(tt)] = valid ? cscale(ld_c<TI>(src, tt), -sgnf(tt)) : make_float2(0.f, 0.f);
   }
   __syncthreads();
   fft_lds<N, E, false>(s, t, twr);
-  if (valid) {
-    for (int e = 0; e < E; ++e) {
-      const int tt = t + e * T;
-      const float sc = a.filt ? -sgnf(tt) * a.filt[tt] : -sgnf(tt);
-      a.Sh[((int64_t)th * N + tt) * a.nz + z] = cscale(s[fpad(tt)], sc);
-    }
+  const int c = threadIdx.x % C, p0 = threadIdx.x / C;
+  if (l0 + c >= lines) return;
+  const LineIdx li(a, l0 + c);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int tt = p0 + e * T;
+    const float sc = a.filt ? -sgnf(tt) * a.filt[tt] : -sgnf(tt);
+    a.Sh[li.at(tt)] = cscale(lds[c * LS + fpad(tt)], sc);
   }
 }
 
@@ -341,10 +436,6 @@ __global__ __launch_bounds__(256) void tomo_filter_k(const TIO* in, TIO* out, in
 constexpr int kHeavyTile = 128;
 constexpr int kLongTile = 512;  // from here more wavefronts share a long list (few slices)
 constexpr int kBatch = 4;  // steps of four samples taken together
-constexpr int kWRow = 16;  // a sample's weights along an axis: 3 zeros, 9 taps, 4 zeros
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(8)));  // an odd slice count leaves rows 8-byte aligned
 
 template <int VEC, int U, int NW>
 __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
@@ -646,15 +737,15 @@ struct TomoLineIfftAny {  // line = theta nz + z, length n
   static constexpr bool kInv = true, kTwo = false;
   TomoArgs a;
   TO* out;
-  __device__ float2 load(int64_t line, int, int t) const { return a.Sh[line * a.n + t]; }
+  __device__ float2 load(int64_t line, int, int t) const { return a.Sh[LineIdx(a, line).at(t)]; }
   __device__ void mid(float2*, int64_t, int, int, int) const {}
   __device__ void store(int64_t line, int, int t, float2 v) const {
-    st_c<TO>(out + line * a.n, t, cscale(v, -sgnf(t) / (4.0f * a.n)));
+    st_c<TO>(out + line * a.n, t, cscale(v, -sgnf(t) * (float)(0.25 / ((double)a.n * a.n))));
   }
 };
 
 template <typename TI>
-struct TomoLineFftAny {  // line = theta nz + z, length n; z-contiguous output
+struct TomoLineFftAny {  // line = theta nz + z, length n; slices-fastest output
   static constexpr bool kInv = false, kTwo = false;
   TomoArgs a;
   const TI* data;
@@ -663,9 +754,8 @@ struct TomoLineFftAny {  // line = theta nz + z, length n; z-contiguous output
   }
   __device__ void mid(float2*, int64_t, int, int, int) const {}
   __device__ void store(int64_t line, int, int t, float2 v) const {
-    const int64_t th = line / a.nz, z = line % a.nz;
     const float sc = a.filt ? -sgnf(t) * a.filt[t] : -sgnf(t);
-    a.Sh[(th * a.n + t) * a.nz + z] = cscale(v, sc);
+    a.Sh[LineIdx(a, line).at(t)] = cscale(v, sc);
   }
 };
 
@@ -733,9 +823,7 @@ static hipError_t tomo_fwd_any(const TomoArgs& a, const TIO* obj, TIO* out, hipS
   if (e != hipSuccess) return e;
   const int C = any_cols_c(N2, any_max_lds()), groups = (N2 + C - 1) / C;
   if ((e = any_launch_cols(TomoColsFwdAny{a, C, groups}, f2, C, (int64_t)a.nz * groups, st)) != hipSuccess) return e;
-  hipLaunchKernelGGL(tomo_tile_gather_k, dim3((unsigned)a.nitems, (unsigned)((a.nz + kTZ - 1) / kTZ)), dim3(256), 0,
-                     st, a);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if ((e = launch_gather(a, st)) != hipSuccess) return e;
   return any_launch_rows(TomoLineIfftAny<TIO>{a, out}, f1, (int64_t)a.ntheta * a.nz, st);
 }
 
@@ -777,14 +865,15 @@ static hipError_t tomo_fwd_n(const TomoArgs& a, const TIO* obj, TIO* out, hipStr
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((tomo_cols_fwd_k<N2, E, C>), dim3((unsigned)(a.nz * (N2 / C))), dim3(C * (N2 / E)), 0, st, a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  constexpr int EL = N >= 8 ? 8 : N;
-  constexpr int RL = 256 / (N / EL);
+  if ((e = launch_gather(a, st)) != hipSuccess) return e;
+  constexpr int EL = N >= 8 ? 8 : N, CL = line_c<N>();
   const int64_t lines = (int64_t)a.ntheta * a.nz;
-  hipLaunchKernelGGL(tomo_tile_gather_k, dim3((unsigned)a.nitems, (unsigned)((a.nz + kTZ - 1) / kTZ)), dim3(256), 0,
-                     st, a);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL((tomo_line_ifft_k<N, EL, TIO>), dim3((unsigned)((lines + RL - 1) / RL)), dim3(256), 0, st, a,
-                     out);
+  if (lines < kLineFew)
+    hipLaunchKernelGGL((tomo_line_ifft_k<N, EL, 4, TIO>), dim3((unsigned)((lines + 3) / 4)), dim3(4 * (N / EL)), 0,
+                       st, a, out);
+  else
+    hipLaunchKernelGGL((tomo_line_ifft_k<N, EL, CL, TIO>), dim3((unsigned)((lines + CL - 1) / CL)),
+                       dim3(CL * (N / EL)), 0, st, a, out);
   return hipGetLastError();
 }
 
@@ -792,11 +881,14 @@ template <int N2, typename TIO>
 static hipError_t tomo_adj_n(const TomoArgs& a, const TIO* data, TIO* out, hipStream_t st) {
   constexpr int E = 8, N = N2 / 2;
   constexpr int C = tomo_cols_c<N2>();
-  constexpr int EL = N >= 8 ? 8 : N;
-  constexpr int RL = 256 / (N / EL);
+  constexpr int EL = N >= 8 ? 8 : N, CL = line_c<N>();
   const int64_t lines = (int64_t)a.ntheta * a.nz;
-  hipLaunchKernelGGL((tomo_linefft_k<N, EL, TIO>), dim3((unsigned)((lines + RL - 1) / RL)), dim3(256), 0, st, a,
-                     data);
+  if (lines < kLineFew)
+    hipLaunchKernelGGL((tomo_linefft_k<N, EL, 4, TIO>), dim3((unsigned)((lines + 3) / 4)), dim3(4 * (N / EL)), 0, st,
+                       a, data);
+  else
+    hipLaunchKernelGGL((tomo_linefft_k<N, EL, CL, TIO>), dim3((unsigned)((lines + CL - 1) / CL)),
+                       dim3(CL * (N / EL)), 0, st, a, data);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if ((e = launch_grid_gather(a, st)) != hipSuccess) return e;
@@ -871,10 +963,10 @@ struct htamd_tomo_plan {
   int* tp = nullptr;
   int2* te = nullptr;
   int4* items = nullptr;
-  int2* so = nullptr;
-  float2* sf = nullptr;
+  int2* ge = nullptr;
+  int* gc = nullptr;
   int* heavy = nullptr;
-  int nitems = 0, ts = 0, nheavy = 0, longest = 0;
+  int nitems = 0, nheavy = 0, longest = 0, sparse = 0;
   // detector filters (ramp, Shepp-Logan, Parzen): [3][n] with the 1/n of the
   // inverse transform for htamd_tomo_filter, and [3][n] shifted by n/2 and
   // scaled by sqrt(n / ntheta) for htamd_tomo_fbp
@@ -991,37 +1083,60 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
   std::stable_sort(heavy.begin(), heavy.end(), [&](int x, int y) {
     return tp[(size_t)x + 1] - tp[(size_t)x] > tp[(size_t)y + 1] - tp[(size_t)y];
   });
-  // Tile binning of the samples for the forward gather: tile of the window's
-  // first tap (wrapped), sorted by tile (counting sort, samples in increasing
-  // order within a tile), cut into work items of at most 256 samples.
-  const int ts = (int)std::min<int64_t>(32, n2);
-  const int ntx = (int)((n2 + ts - 1) / ts);  // the last tile is partial when ts does not divide 2n
-  std::vector<int> tcount((size_t)(ntx * ntx + 1), 0);
-  for (int64_t si = 0; si < S; ++si)
-    ++tcount[(size_t)((wrap(tb[(size_t)si].y) / ts) * ntx + wrap(tb[(size_t)si].x) / ts + 1)];
-  for (int i = 0; i < ntx * ntx; ++i) tcount[(size_t)(i + 1)] += tcount[(size_t)i];
-  std::vector<int> tfill(tcount.begin(), tcount.end() - 1);
-  std::vector<int2> so((size_t)S);
-  std::vector<float2> sf((size_t)S);
-  for (int64_t si = 0; si < S; ++si) {
+  // The samples by region and cell of the window's first tap (wrapped), for the
+  // forward gather (counting sort, samples in increasing order within a cell),
+  // each cell's cut into groups of 16 and each region's groups into work items.
+  const int nr = (int)((n2 + kRG - 1) / kRG);  // the last region is partial when kRG does not divide 2n
+  constexpr int kCX = kRG / kCellX, kCells = kCX * (kRG / kCellY);
+  auto cell_of = [&](int64_t si) {
     const int wx0 = wrap(tb[(size_t)si].x), wy0 = wrap(tb[(size_t)si].y);
-    const int tile = (wy0 / ts) * ntx + wx0 / ts;
-    const int k = tfill[(size_t)tile]++;
-    so[(size_t)k] = make_int2(((wy0 % ts) << 16) | (wx0 % ts), (int)si);
-    const int64_t kk = si / n, t = si % n;
-    const double th = (double)(float)theta[kk];
-    const double x2 = (double)n2 * ((double)(t - n / 2) / (double)n * std::cos(th));
-    const double y2 = (double)n2 * (-(double)(t - n / 2) / (double)n * std::sin(th));
-    sf[(size_t)k] = make_float2((float)(x2 - std::floor(x2)), (float)(y2 - std::floor(y2)));
+    return ((wy0 / kRG) * nr + wx0 / kRG) * kCells + wy0 % kRG / kCellY * kCX + wx0 % kRG / kCellX;
+  };
+  std::vector<int> ccount((size_t)nr * nr * kCells, 0);
+  for (int64_t si = 0; si < S; ++si) ++ccount[(size_t)cell_of(si)];
+  // steps of four points of either form, staging a region counted as kStageSteps
+  int64_t dense = 0, sparse = 0;
+  for (int rg = 0; rg < nr * nr; ++rg) {
+    int sum = 0, groups = 0;
+    for (int c = 0; c < kCells; ++c) {
+      const int k = ccount[(size_t)(rg * kCells + c)];
+      groups += (k + 15) / 16;
+      sum += k;
+    }
+    using D = GatherShape<false>;
+    using P = GatherShape<true>;
+    dense += groups * D::NY * D::NX + (groups + kItemGroups - 1) / kItemGroups * kStageSteps;
+    sparse += (sum + 15) / 16 * (P::NY * P::NX + kStageSteps);
   }
+  p->sparse = sparse < dense;
+  std::vector<int> cfill(ccount.size());
+  std::vector<int> gc;
   std::vector<int4> items;
-  for (int tile = 0; tile < ntx * ntx; ++tile)
-    for (int b = tcount[(size_t)tile]; b < tcount[(size_t)(tile + 1)]; b += 256)
-      items.push_back(make_int4(tile % ntx, tile / ntx, b, std::min(256, tcount[(size_t)(tile + 1)] - b)));
+  for (int rg = 0; rg < nr * nr; ++rg) {
+    const int first = (int)gc.size();
+    for (int c = 0, fill = 0; c < kCells; ++c) {
+      const int k = ccount[(size_t)(rg * kCells + c)];
+      if (p->sparse) {
+        cfill[(size_t)(rg * kCells + c)] = 16 * first + fill;
+        fill += k;
+        while (16 * ((int)gc.size() - first) < fill) gc.push_back(0);
+      } else {
+        cfill[(size_t)(rg * kCells + c)] = 16 * (int)gc.size();
+        for (int i = 0; i < k; i += 16) gc.push_back(c / kCX << 8 | c % kCX);
+      }
+    }
+    const int step = p->sparse ? 1 : kItemGroups;
+    for (int b = first; b < (int)gc.size(); b += step)
+      items.push_back(make_int4(rg % nr, rg / nr, b, std::min(step, (int)gc.size() - b)));
+  }
+  std::vector<int2> ge(16 * gc.size(), make_int2(-1, 0));
+  const int py = p->sparse ? kRG : kCellY, px = p->sparse ? kRG : kCellX;
+  for (int64_t si = 0; si < S; ++si)
+    ge[(size_t)cfill[(size_t)cell_of(si)]++] =
+        make_int2((int)si, wrap(tb[(size_t)si].y) % kRG % py << 8 | wrap(tb[(size_t)si].x) % kRG % px);
   p->nitems = (int)items.size();
   p->nheavy = (int)heavy.size();
   p->longest = heavy.empty() ? 0 : tp[(size_t)heavy[0] + 1] - tp[(size_t)heavy[0]];
-  p->ts = ts;
   // deapodiser phi (tomo.py:19-21, 46-47) with the mask folded in
   std::vector<float> phi((size_t)(n * n));
   for (int64_t i = 0; i < n; ++i) {
@@ -1059,7 +1174,7 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
       (e = up(&p->tp, tp)) != hipSuccess || (e = up(&p->te, te)) != hipSuccess ||
       (e = up(&p->items, items)) != hipSuccess ||
       (!heavy.empty() && (e = up(&p->heavy, heavy)) != hipSuccess) ||
-      (e = up(&p->so, so)) != hipSuccess || (e = up(&p->sf, sf)) != hipSuccess ||
+      (e = up(&p->ge, ge)) != hipSuccess || (e = up(&p->gc, gc)) != hipSuccess ||
       (e = up(&p->filt, filt)) != hipSuccess || (e = up(&p->filt_fbp, filt_fbp)) != hipSuccess) {
     htamd_tomo_plan_destroy(p);
     return hip_fail(e, "tomo_plan_create");
@@ -1077,8 +1192,8 @@ int htamd_tomo_plan_destroy(htamd_tomo_plan* p) {
   (void)hipFree(p->tp);
   (void)hipFree(p->te);
   (void)hipFree(p->items);
-  (void)hipFree(p->so);
-  (void)hipFree(p->sf);
+  (void)hipFree(p->ge);
+  (void)hipFree(p->gc);
   (void)hipFree(p->heavy);
   (void)hipFree(p->filt);
   (void)hipFree(p->filt_fbp);
@@ -1117,15 +1232,13 @@ static int tomo_run(const htamd_tomo_plan* p, bool adjoint, const void* in, int 
   a.tw2 = p->tw2;
   a.tw1 = p->tw1;
   a.items = p->items;
-  a.so = p->so;
-  a.sf = p->sf;
-  a.ts = p->ts;
+  a.ge = p->ge;
+  a.gc = p->gc;
   a.nitems = p->nitems;
+  a.sparse = p->sparse;
   a.heavy = p->heavy;
   a.nheavy = p->nheavy;
   a.longest = p->longest;
-  a.cxs = (float)(-M_PI * M_PI / p->mu / (4.0 * (double)p->n * (double)p->n));
-  a.cys = (float)(M_PI / p->mu);
   a.W = (float2*)ws;
   a.G = (float2*)ws + nz * p->n * 2 * p->n;
   a.Sh = a.G + nz * 4 * p->n * p->n;

@@ -50,3 +50,32 @@ def test_factorisation_orders_radices(checker):
     assert rad[6528] == [8, 8, 2, 3, 17]
     assert rad[2500] == [4, 5, 5, 5, 5]
     assert rad[1536] == [8, 8, 8, 3]
+
+
+@pytest.mark.parametrize("lengths", [(11, 13, 77, 143, 182, 286, 1001), (19, 23, 38, 289, 361, 458, 2058, 4370)])
+def test_prime_radices_match_direct_dft(checker, lengths):
+    """In-register radices 7, 11 and 13, and direct stages of larger primes:
+    alone, after other stages (twiddled), twice, and with an odd and an even
+    number of output pairs."""
+    out = subprocess.run([checker] + [str(n) for n in lengths], capture_output=True, text=True, check=True).stdout
+    rows = [line.split() for line in out.strip().splitlines()]
+    assert [int(r[0]) for r in rows] == list(lengths)
+    for r in rows:
+        assert float(r[1]) < 5e-7 and float(r[2]) < 5e-7, r
+
+
+def test_division_by_multiplication(tmp_path):
+    """AnyMod's quotients and remainders for every length of a line that fits the
+    LDS and every divisor of a stage below it."""
+    if not (os.path.exists(HIPCC) or shutil.which("hipcc")):
+        pytest.skip("hipcc not available")
+    src = tmp_path / "mod.cpp"
+    src.write_text('#include <cstdio>\n#include "fft_any.hpp"\n'
+                   "int main() { long bad = 0; for (int d = 1; d <= 10240; ++d) { htamd::AnyMod m(d);\n"
+                   "  for (int j = 0; j <= 20480; j += (j % d > 1 && j % d < d - 2) ? d - 2 - j % d : 1)\n"
+                   "    bad += m.div(j) != j / d || m(j) != j % d; }\n"
+                   'std::printf("%ld\\n", bad); return bad != 0; }\n')
+    exe = str(tmp_path / "mod")
+    subprocess.run([HIPCC, "-O2", "-std=c++17", "--offload-arch=gfx950", "-I" + CSRC, str(src), "-o", exe],
+                   check=True, capture_output=True)
+    assert subprocess.run([exe], capture_output=True, text=True, check=True).stdout.strip() == "0"

@@ -136,3 +136,20 @@ def test_bh_loop_any_size_matches_oracle(gpu):
         assert errs[k] == pytest.approx(hist[k][2], rel=1e-4)
     for k in ("obj", "prb", "pos"):
         assert rel(rec.vars[k], vo[k]) < 1e-4, k
+
+
+@pytest.mark.parametrize("n,nz,B", [(14, 22, 3), (26, 286, 2), (34, 38, 2), (300, 640, 1), (298, 642, 1), (18, 2560, 1),
+                                    (10, 5120, 1), (22, 5122, 1), (8, 8190, 1)])
+def test_D_DT_column_tiles_and_prime_radices(gpu, n, nz, B):
+    """Column tiles of 16 down to 1 lines (the sizes at which two workgroups no
+    longer fit the LDS, and the largest), row lengths they do not divide, and
+    lengths with prime factors 7 to 197.  The sum of the squares of a line's
+    stage errors keeps these at the bar of the other sizes."""
+    from holotomocupy_amd import Propagation
+    print(f"[case] D/DT column tiles n={n} nz={nz}", flush=True)
+    rng = np.random.default_rng(n + nz)
+    g, o = Propagation(n, nz, B, 1, 1.0, 1.0, [1e3]), op.Propagation(n, nz, B, 1, 1.0, 1.0, [1e3])
+    x = crandn(rng, (B, nz, n))
+    xt = torch.from_numpy(x).to(gpu)
+    assert rel(g.D(xt, 0), o.D(x.astype(np.complex128), 0)) < REL_TOL
+    assert rel(g.DT(xt, 0), o.DT(x.astype(np.complex128), 0)) < REL_TOL

@@ -474,103 +474,47 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
 }
 
 // ---- K4: gather-form Sadj summed over distances ----------------------------
-// K4: dpsi = rho_obj * sum_j Sadj_j(T_j) as a gather.  A workgroup owns a
-// 64 x kSadjTY tile of coefficients: lane l of wave w computes column l of rows
-// w*kSadjR .. w*kSadjR + kSadjR - 1, so its x weights serve kSadjR outputs and
-// a wave's rows are wave-uniform.  For a distance with magnification >= 1
-// every candidate bracket has fewer than 8 entries; the tile's y weights
-// (kSadjTY rows x 8 candidates) are then evaluated once into LDS and read as
-// broadcasts.  Smaller magnifications take the per-thread candidate walk.
-// Either way each output sums over detector rows in ascending order and the
-// distances in order.
-constexpr int kSadjR = 4, kSadjTY = 4 * kSadjR, kSadjK = 8;
-
+// dpsi = rho_obj * sum_j Sadj_j(T_j) on tiles of 64 x kAtY coefficients: a
+// distance with magnification >= 1 through LDS (adj_tile_add), a smaller one by
+// walking the candidates of each output.  Each output sums over detector rows in
+// ascending order and the distances in order.
+// 16 angles of 1024^2 from 4 distances of 2048^2: 512 us walking the candidates
+// -> 306 us; 48 angles of 256^2 from 2 distances 69 -> 39 us.
 template <typename TO>
-__global__ __launch_bounds__(256) void bh_sadj_k(BhArgs a, TO* __restrict__ dpsi, int tiles_x,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void bh_sadj_k(BhArgs a, TO* __restrict__ dpsi, int tiles_x,
                                                  int tiles_y) {
-  constexpr int TX = 64, R = kSadjR, TY = kSadjTY, K = kSadjK;
-  __shared__ float s_wy[TY][K];
-  __shared__ int s_ylo[TY];
+  __shared__ AdjTile<TO> tile;
   const int64_t bid = xcd_tile(blockIdx.x, gridDim.x);
   const int txt = (int)(bid % tiles_x);
   const int64_t rest = bid / tiles_x;
   const int tyt = (int)(rest % tiles_y);
   const int64_t b = rest / tiles_y;
   const int t = threadIdx.x;
-  const int ix = txt * TX + (t & 63);
-  const int r0 = (t >> 6) * R;  // first tile row of this wave
+  const int ix0 = txt * kAtX, iy0 = tyt * kAtY;
+  const int ix = ix0 + (t & 63), iy = iy0 + (t >> 6) * kAtR;
   const bool xin = ix < a.npsi;
-  TO acc[R];
+  TO acc[kAtR];
 #pragma unroll
-  for (int rr = 0; rr < R; ++rr) acc[rr] = vzero<TO>();
+  for (int rr = 0; rr < kAtR; ++rr) acc[rr] = vzero<TO>();
+  adj_tile_init(tile);
+#pragma unroll 1
   for (int j = 0; j < a.ndist; ++j) {
     const int64_t bj = b * a.ndist + j;
     const float mb = a.mag[bj], ry = a.pos[2 * bj], rx = a.pos[2 * bj + 1];
     const float2* g = a.T + bj * (int64_t)a.nz * a.n;
     if (mb >= 1.0f) {  // uniform over the workgroup (one angle)
-      __syncthreads();  // the previous distance's table has been read
-      if (t < TY * K) {
-        const int row = t / K, k = t % K, iy = tyt * TY + row;
-        float w = 0.0f;
-        int ylo = 0, yhi = -1;
-        if (iy < a.nzpsi) {
-          bs_candidates(iy, a.nz, a.nzpsi, mb, ry, ylo, yhi);
-          if (ylo + k <= yhi) w = bs_reach(bs_pos(ylo + k, a.nz, a.nzpsi, mb, ry), iy);
-        }
-        s_wy[row][k] = w;
-        if (k == 0) s_ylo[row] = ylo;
-      }
-      __syncthreads();
-      if (xin) {
-        int xlo, xhi;
-        bs_candidates(ix, a.n, a.npsi, mb, rx, xlo, xhi);
-        float wxs[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-          wxs[k] = xlo + k <= xhi ? bs_reach(bs_pos(xlo + k, a.n, a.npsi, mb, rx), ix) : 0.0f;
-        // the R outputs' candidate detector rows overlap: walk their union in
-        // ascending order, form each row's x sum once and add it to every
-        // output that weights it (per output the same terms in the same order)
-        // over the rows that exist (rows past the plane have no candidates)
-        int ylo = INT_MAX, yhi = INT_MIN;
-#pragma unroll
-        for (int rr = 0; rr < R; ++rr) {
-          if (tyt * TY + r0 + rr >= a.nzpsi) continue;
-          ylo = min(ylo, s_ylo[r0 + rr]);
-          yhi = max(yhi, s_ylo[r0 + rr]);
-        }
-        yhi += K - 1;
-        for (int ty = ylo; ty <= yhi; ++ty) {
-          float wv[R];
-          bool any = false;
-#pragma unroll
-          for (int rr = 0; rr < R; ++rr) {
-            const int d = ty - s_ylo[r0 + rr];
-            wv[rr] = d >= 0 && d < K ? s_wy[r0 + rr][d] : 0.0f;
-            any = any || wv[rr] != 0.0f;
-          }
-          if (!any) continue;  // wave-uniform: the rows are the wave's
-          const float2* gr = g + (int64_t)ty * a.n + xlo;
-          TO rowv = vzero<TO>();
-#pragma unroll
-          for (int kk = 0; kk < K; ++kk)
-            if (wxs[kk] != 0.0f) rowv = vfma(wxs[kk], from_c<TO>(gr[kk]), rowv);
-#pragma unroll
-          for (int rr = 0; rr < R; ++rr)
-            if (wv[rr] != 0.0f) acc[rr] = vfma(wv[rr], rowv, acc[rr]);
-        }
-      }
+      adj_tile_add(tile, ix0, iy0, a.n, a.nz, a.npsi, a.nzpsi, mb, rx, ry,
+                   [&](int ty, int tx) { return from_c<TO>(g[(int64_t)ty * a.n + tx]); }, acc);
     } else if (xin) {
       int xlo, xhi;
       bs_candidates(ix, a.n, a.npsi, mb, rx, xlo, xhi);
 #pragma unroll
-      for (int rr = 0; rr < R; ++rr) {
-        const int iy = tyt * TY + r0 + rr;
-        if (iy >= a.nzpsi) continue;
+      for (int rr = 0; rr < kAtR; ++rr) {
+        if (iy + rr >= a.nzpsi) continue;
         int ylo, yhi;
-        bs_candidates(iy, a.nz, a.nzpsi, mb, ry, ylo, yhi);
+        bs_candidates(iy + rr, a.nz, a.nzpsi, mb, ry, ylo, yhi);
         for (int ty = ylo; ty <= yhi; ++ty) {
-          const float wyv = bs_reach(bs_pos(ty, a.nz, a.nzpsi, mb, ry), iy);
+          const float wyv = bs_reach(bs_pos(ty, a.nz, a.nzpsi, mb, ry), iy + rr);
           if (wyv == 0.0f) continue;
           TO rowv = vzero<TO>();
           for (int tx = xlo; tx <= xhi; ++tx) {
@@ -585,10 +529,8 @@ __global__ __launch_bounds__(256) void bh_sadj_k(BhArgs a, TO* __restrict__ dpsi
   if (!xin) return;
   const float rho = a.scales[b].y;
 #pragma unroll
-  for (int rr = 0; rr < R; ++rr) {
-    const int iy = tyt * TY + r0 + rr;
-    if (iy < a.nzpsi) dpsi[(b * a.nzpsi + iy) * (int64_t)a.npsi + ix] = vfma(rho, acc[rr], vzero<TO>());
-  }
+  for (int rr = 0; rr < kAtR; ++rr)
+    if (iy + rr < a.nzpsi) dpsi[(b * a.nzpsi + iy + rr) * (int64_t)a.npsi + ix] = vfma(rho, acc[rr], vzero<TO>());
 }
 
 // ---- small reductions -------------------------------------------------------
@@ -892,7 +834,7 @@ static hipError_t bh_run(const htamd_shift_plan* sp, BhArgs a, const void* proj,
   sev.mark(6, st);
   if ((e = rows_dispatch<TO>(true, a, st)) != hipSuccess) return e;
   sev.mark(7, st);
-  const int tx = (a.npsi + 63) / 64, ty = (a.nzpsi + kSadjTY - 1) / kSadjTY;
+  const int tx = (a.npsi + kAtX - 1) / kAtX, ty = (a.nzpsi + kAtY - 1) / kAtY;
   TO* dpsi = (TO*)(ws + L.dpsi);
   sev.mark(8, st);
   hipLaunchKernelGGL((bh_sadj_k<TO>), dim3((unsigned)(a.nang * tx * ty)), dim3(256), 0, st, a, dpsi, tx, ty);

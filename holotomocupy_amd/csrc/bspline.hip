@@ -186,100 +186,44 @@ __global__ __launch_bounds__(256) void bs_interp_rows_k(BsArgs<T> a) {
 //   sum_{ty: iy in taps(y(ty))} wy(ty) sum_{tx: ix in taps(x(tx))} wx(tx) g[b, ty, tx].
 // Candidate pixels are bracketed analytically with a one-pixel margin and each
 // is re-evaluated with the forward's exact float expression, so the weights
-// are bitwise those of S.  Tiles of 64 x kAdjTY coefficients: lane l of wave w
-// computes column l of rows w*kAdjR .. w*kAdjR + kAdjR - 1, so its x weights
-// serve kAdjR outputs.  With magnification >= 1 every candidate bracket holds
-// fewer than 8 entries (an entry past 8 is the outer margin, whose weight is
-// zero), and the tile's y weights are evaluated once into LDS; smaller
-// magnifications walk the brackets per thread.  Each output sums detector rows
-// in ascending order either way.
-constexpr int kAdjR = 4, kAdjTY = 4 * kAdjR, kAdjK = 8;
-
+// are bitwise those of S.  A workgroup takes a tile of 64 x kAtY coefficients:
+// with magnification >= 1 through LDS (adj_tile_add), else (wider brackets) each
+// thread walks the candidates of its kAtR rows of one column.  Each output sums
+// detector rows in ascending order either way.
+// 384 planes of 256^2: 269 us walking the candidates -> 141 us (both planes
+// move once: 78 us at the card's copy rate).
 template <typename T>
 __global__ __launch_bounds__(256) void bs_adjoint_k(BsArgs<T> a) {
   // here a.c is the input g [B, nz, n] and a.out the coefficients [B, nzpsi, npsi]
-  constexpr int R = kAdjR, TY = kAdjTY, K = kAdjK;
-  __shared__ float s_wy[TY][K];
-  __shared__ int s_ylo[TY];
-  const int64_t bid = blockIdx.x;
+  __shared__ AdjTile<T> tile;
+  const int64_t bid = xcd_tile(blockIdx.x, gridDim.x);
   const int txt = (int)(bid % a.tiles_x);
   const int64_t rest = bid / a.tiles_x;
   const int tyt = (int)(rest % a.tiles_y);
   const int64_t b = rest / a.tiles_y;
   const int t = threadIdx.x;
-  const int ix = txt * 64 + (t & 63);
-  const int r0 = (t >> 6) * R;
-  const bool xin = ix < a.npsi;
+  const int ix0 = txt * kAtX, iy0 = tyt * kAtY;
+  const int ix = ix0 + (t & 63), iy = iy0 + (t >> 6) * kAtR;
   const float mb = a.m[b * a.ms];
   const float rx = a.r[b * a.rs + 1], ry = a.r[b * a.rs + 0];
   const T* g = a.c + b * (int64_t)a.nz * a.n;
-  T acc[R];
+  T acc[kAtR];
 #pragma unroll
-  for (int rr = 0; rr < R; ++rr) acc[rr] = vzero<T>();
+  for (int rr = 0; rr < kAtR; ++rr) acc[rr] = vzero<T>();
   if (mb >= 1.0f) {  // uniform over the workgroup (one angle)
-    if (t < TY * K) {
-      const int row = t / K, k = t % K, iy = tyt * TY + row;
-      float w = 0.0f;
-      int ylo = 0, yhi = -1;
-      if (iy < a.nzpsi) {
-        bs_candidates(iy, a.nz, a.nzpsi, mb, ry, ylo, yhi);
-        if (ylo + k <= yhi) w = bs_reach(bs_pos(ylo + k, a.nz, a.nzpsi, mb, ry), iy);
-      }
-      s_wy[row][k] = w;
-      if (k == 0) s_ylo[row] = ylo;
-    }
-    __syncthreads();
-    if (xin) {
-      int xlo, xhi;
-      bs_candidates(ix, a.n, a.npsi, mb, rx, xlo, xhi);
-      float wxs[K];
-#pragma unroll
-      for (int k = 0; k < K; ++k)
-        wxs[k] = xlo + k <= xhi ? bs_reach(bs_pos(xlo + k, a.n, a.npsi, mb, rx), ix) : 0.0f;
-      // the R outputs' candidate detector rows overlap (three of four at
-      // magnification 1): walk their union in ascending order, form each
-      // row's x sum once and add it to every output that weights it -- per
-      // output the same terms in the same order as a walk of its own rows
-      // over the rows that exist (rows past the plane have no candidates)
-      int ylo = INT_MAX, yhi = INT_MIN;
-#pragma unroll
-      for (int rr = 0; rr < R; ++rr) {
-        if (tyt * TY + r0 + rr >= a.nzpsi) continue;
-        ylo = min(ylo, s_ylo[r0 + rr]);
-        yhi = max(yhi, s_ylo[r0 + rr]);
-      }
-      yhi += K - 1;
-      for (int ty = ylo; ty <= yhi; ++ty) {
-        float wv[R];
-        bool any = false;
-#pragma unroll
-        for (int rr = 0; rr < R; ++rr) {
-          const int d = ty - s_ylo[r0 + rr];
-          wv[rr] = d >= 0 && d < K ? s_wy[r0 + rr][d] : 0.0f;
-          any = any || wv[rr] != 0.0f;
-        }
-        if (!any) continue;  // wave-uniform: the rows are the wave's
-        const T* gr = g + (int64_t)ty * a.n + xlo;
-        T row = vzero<T>();
-#pragma unroll
-        for (int kk = 0; kk < K; ++kk)
-          if (wxs[kk] != 0.0f) row = vfma(wxs[kk], gr[kk], row);
-#pragma unroll
-        for (int rr = 0; rr < R; ++rr)
-          if (wv[rr] != 0.0f) acc[rr] = vfma(wv[rr], row, acc[rr]);
-      }
-    }
-  } else if (xin) {
+    adj_tile_init(tile);
+    adj_tile_add(tile, ix0, iy0, a.n, a.nz, a.npsi, a.nzpsi, mb, rx, ry,
+                 [&](int ty, int tx) { return g[(int64_t)ty * a.n + tx]; }, acc);
+  } else if (ix < a.npsi) {
     int xlo, xhi;
     bs_candidates(ix, a.n, a.npsi, mb, rx, xlo, xhi);
 #pragma unroll
-    for (int rr = 0; rr < R; ++rr) {
-      const int iy = tyt * TY + r0 + rr;
-      if (iy >= a.nzpsi) continue;
+    for (int rr = 0; rr < kAtR; ++rr) {
+      if (iy + rr >= a.nzpsi) continue;
       int ylo, yhi;
-      bs_candidates(iy, a.nz, a.nzpsi, mb, ry, ylo, yhi);
+      bs_candidates(iy + rr, a.nz, a.nzpsi, mb, ry, ylo, yhi);
       for (int ty = ylo; ty <= yhi; ++ty) {
-        const float wyv = bs_reach(bs_pos(ty, a.nz, a.nzpsi, mb, ry), iy);
+        const float wyv = bs_reach(bs_pos(ty, a.nz, a.nzpsi, mb, ry), iy + rr);
         if (wyv == 0.0f) continue;
         T row = vzero<T>();
         for (int tx = xlo; tx <= xhi; ++tx) {
@@ -290,12 +234,10 @@ __global__ __launch_bounds__(256) void bs_adjoint_k(BsArgs<T> a) {
       }
     }
   }
-  if (!xin) return;
+  if (ix >= a.npsi) return;
 #pragma unroll
-  for (int rr = 0; rr < R; ++rr) {
-    const int iy = tyt * TY + r0 + rr;
-    if (iy < a.nzpsi) a.out[(b * a.nzpsi + iy) * (int64_t)a.npsi + ix] = acc[rr];
-  }
+  for (int rr = 0; rr < kAtR; ++rr)
+    if (iy + rr < a.nzpsi) a.out[(b * a.nzpsi + iy + rr) * (int64_t)a.npsi + ix] = acc[rr];
 }
 
 // ---------------------------------------------------------------------------
@@ -557,8 +499,8 @@ hipError_t bs_launch_forward(BsArgs<T> a, int mode, hipStream_t st) {
 
 template <typename T>
 hipError_t bs_launch_adjoint(BsArgs<T> a, hipStream_t st) {
-  a.tiles_x = (a.npsi + 63) / 64;
-  a.tiles_y = (a.nzpsi + kAdjTY - 1) / kAdjTY;
+  a.tiles_x = (a.npsi + kAtX - 1) / kAtX;
+  a.tiles_y = (a.nzpsi + kAtY - 1) / kAtY;
   const int64_t grid = a.batch * (int64_t)a.tiles_x * a.tiles_y;
   if (grid == 0) return hipSuccess;
   hipLaunchKernelGGL((bs_adjoint_k<T>), dim3((unsigned)grid), dim3(256), 0, st, a);

@@ -116,6 +116,115 @@ __device__ __forceinline__ float2 block_sum2(float2 v) {
   return s;
 }
 
+// ---- Sadj of one tile of coefficients, magnification >= 1 ------------------------
+// acc[rr] += sum over detector rows ty, then columns tx, of wy wx g[ty][tx] for
+// the coefficients (iy0 + wave kAtR + rr, ix0 + lane) of a 64 x kAtY tile (a
+// workgroup of 256 threads).  The detector pixels that reach the tile are
+// staged in LDS once; each detector row's x sums are formed once and serve all
+// coefficient rows that weigh them, so an output costs about 5 reads for x and
+// 4 for y, all from LDS.  Walking the candidates per output row group read each
+// pixel some 28 times through the L1, eight predicated loads to a row, and waited
+// for each row; here all loads of a tile are in flight together (without that the
+// tile form measured 247 us against the walk's 269, with it 141).
+// Magnification >= 1 leaves at most 4 pixels with a weight along each axis,
+// consecutive ones within the first 8 of the bracket; taps that are not there
+// read a zeroed slot, so nothing else enters the sums, which run in the order of
+// the walk (ascending rows, ascending columns).
+constexpr int kAtX = 64, kAtR = 8, kAtY = 4 * kAtR;
+constexpr int kAtNX = kAtX + 12, kAtNY = kAtY + 12;  // brackets: (tile + 3) / m + 4 and the margins
+
+template <typename TO>
+struct AdjTile {
+  TO g[kAtNY][kAtNX + 1];    // the last column of each row stays zero
+  TO tmp[kAtNY + 1][kAtX];   // x sums; the last row stays zero
+  float wy[kAtY][4];
+  int fy[kAtY];
+};
+
+// 4 consecutive weights w with which index i collects pixels f .. f + 3 (f = -1: none)
+__device__ __forceinline__ int bs_adj_taps(int i, int npix, int npsi, float mb, float r, float (&w)[4]) {
+  int lo, hi, f = -1;
+  bs_candidates(i, npix, npsi, mb, r, lo, hi);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) w[j] = 0.0f;
+#pragma unroll 2
+  for (int k = 0; k < 8; ++k) {
+    const float v = lo + k <= hi ? bs_reach(bs_pos(lo + k, npix, npsi, mb, r), i) : 0.0f;
+    if (f < 0 && v != 0.0f) f = lo + k;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (f >= 0 && lo + k == f + j) w[j] = v;
+  }
+  return f;
+}
+
+// Once per kernel, before the first adj_tile_add (which begins with a barrier).
+template <typename TO>
+__device__ __forceinline__ void adj_tile_init(AdjTile<TO>& s) {
+  if (threadIdx.x < kAtNY) s.g[threadIdx.x][kAtNX] = vzero<TO>();
+  if (threadIdx.x < kAtX) s.tmp[kAtNY][threadIdx.x] = vzero<TO>();
+}
+
+template <typename TO, typename LOAD>
+__device__ __forceinline__ void adj_tile_add(AdjTile<TO>& s, int ix0, int iy0, int n, int nz, int npsi, int nzpsi,
+                                             float mb, float rx, float ry, const LOAD& load, TO (&acc)[kAtR]) {
+  const int t = threadIdx.x, c = t & 63, wv = t >> 6;
+  // detector pixels whose taps can reach the tile
+  int xlo, xhi, ylo, yhi, unused;
+  bs_candidates(ix0, n, npsi, mb, rx, xlo, unused);
+  bs_candidates(min(ix0 + kAtX, npsi) - 1, n, npsi, mb, rx, unused, xhi);
+  bs_candidates(iy0, nz, nzpsi, mb, ry, ylo, unused);
+  bs_candidates(min(iy0 + kAtY, nzpsi) - 1, nz, nzpsi, mb, ry, unused, yhi);
+  const int ncol = min(xhi - xlo + 1, kAtNX), nrow = min(yhi - ylo + 1, kAtNY);
+  __syncthreads();  // the last tile's sums have been read
+  // (a position that is not finite gives a bracket anywhere: only pixels that
+  // exist are read, and those with a weight do).  All loads are issued before
+  // the first is stored.
+  constexpr int NE = kAtNX - 64, NR = kAtNY / 4, NL = (kAtNY * NE + 255) / 256;
+  TO v[NR + NL];
+  auto at = [&](int r, int k) {
+    const unsigned ty = (unsigned)ylo + r, tx = (unsigned)xlo + k;
+    return r < nrow && k < ncol && tx < (unsigned)n && ty < (unsigned)nz ? load((int)ty, (int)tx) : vzero<TO>();
+  };
+#pragma unroll
+  for (int i = 0; i < NR; ++i) v[i] = at(wv + 4 * i, c);
+#pragma unroll
+  for (int i = 0; i < NL; ++i) v[NR + i] = at((t + 256 * i) / NE, 64 + (t + 256 * i) % NE);
+  if (t < kAtY) {
+    float w[4];
+    s.fy[t] = iy0 + t < nzpsi ? bs_adj_taps(iy0 + t, nz, nzpsi, mb, ry, w) : -1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s.wy[t][j] = iy0 + t < nzpsi ? w[j] : 0.0f;
+  }
+  float wx[4];
+  const int fx = bs_adj_taps(min(ix0 + c, npsi - 1), n, npsi, mb, rx, wx);
+  int ox[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ox[j] = wx[j] != 0.0f ? fx - xlo + j : kAtNX;
+#pragma unroll
+  for (int i = 0; i < NR; ++i) s.g[wv + 4 * i][c] = v[i];
+#pragma unroll
+  for (int i = 0; i < NL; ++i)
+    if (t + 256 * i < kAtNY * NE) s.g[(t + 256 * i) / NE][64 + (t + 256 * i) % NE] = v[NR + i];
+  __syncthreads();
+  for (int r = wv; r < nrow; r += 4) {
+    TO sum = vzero<TO>();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sum = vfma(wx[j], s.g[r][ox[j]], sum);
+    s.tmp[r][c] = sum;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int rr = 0; rr < kAtR; ++rr) {
+    const int row = wv * kAtR + rr, f = s.fy[row];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float w = s.wy[row][j];
+      acc[rr] = vfma(w, s.tmp[w != 0.0f ? f - ylo + j : kAtNY][c], acc[rr]);
+    }
+  }
+}
+
 // ---- launch interface ------------------------------------------------------
 template <typename T>
 struct BsArgs {

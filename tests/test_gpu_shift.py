@@ -178,3 +178,35 @@ def test_coeff_wide_planes(gpu, shape, real):
     c = data(rng, shape, real)
     g = Shift(npsi, npsi, nzpsi, nzpsi, "float32" if real else "complex64")
     assert rel(g.coeff(dev(c)).cpu(), osh.coeff(c, real=real)) < REL_TOL
+
+
+@pytest.mark.parametrize("real", [False, True])
+@pytest.mark.parametrize("n,npsi,nz,nzpsi", [(64, 64, 32, 32), (65, 62, 31, 30), (130, 66, 70, 34), (16, 200, 9, 100),
+                                             (200, 128, 96, 64)])
+def test_Sadj_tiles(gpu, real, n, npsi, nz, nzpsi):
+    """Tiles of 64 x 32 coefficients and their remainders, magnifications of
+    exactly one (integer and fractional shifts), above and below it in one call,
+    shifts that leave tiles partly or wholly without detector pixels, and a
+    value that is not finite, which only the coefficients it reaches see."""
+    from holotomocupy_amd import Shift
+    print(f"[case] Sadj tiles n={n} npsi={npsi} nz={nz} nzpsi={nzpsi} real={real}", flush=True)
+    rng = np.random.default_rng(n + npsi)
+    dt = "float32" if real else "complex64"
+    m = np.array([1, 1, 1.85, 3.2, 0.7, 1, 1.0001], np.float32)
+    r = np.array([[0, 0], [0.3, -2.7], [1.5, 4.25], [-6, 2], [2, -3], [70, -90], [-40.5, 33]], np.float32)
+    B = len(m)
+    g, o = Shift(n, npsi, nz, nzpsi, dt), osh.Shift(n, npsi, nz, nzpsi, dt)
+    s = data(rng, (B, nz, n), real)
+    out, ref = g.Sadj(dev(s), dev(r), dev(m)).cpu().numpy(), o.Sadj(s, r, m)
+    for b in range(B):
+        if np.linalg.norm(ref[b]):
+            assert rel(out[b], ref[b]) < REL_TOL, b
+        else:
+            assert not out[b].any(), b
+    s[:, nz // 2, n // 2] = np.inf
+    mark = np.zeros((B, nz, n), np.float32)
+    mark[:, nz // 2, n // 2] = 1
+    reach = o.Sadj(mark if real else mark.astype(np.complex64), r, m) != 0
+    out2 = g.Sadj(dev(s), dev(r), dev(m)).cpu().numpy()
+    assert np.array_equal(np.isfinite(out2), ~reach)
+    assert np.array_equal(out2[~reach], out[~reach])

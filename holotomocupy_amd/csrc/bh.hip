@@ -172,6 +172,7 @@ __device__ __forceinline__ float2 row_sum2(float2 v, float2* red) {
 template <int N, int E, typename TO, bool STAGED>
 __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(4))) void bh_fwd_rows_k(BhArgs a) {
   constexpr int T = N / E, ROWS = kRowThreads / T;
+  constexpr bool kWave = wave_private<N, E>();  // a row's buffers are one wavefront's
   __shared__ float2 lds[ROWS * fft_buf<N>()];
   const int r = threadIdx.x / T, t0 = threadIdx.x % T;
   const int64_t nunits = (int64_t)a.ndist * a.nz;
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(4))
       int lo, hi;
       row_span<N>(a.npsi, mb, rx, lo, hi);
       stage_row<TO, T, false>(cb, a.npsi, a.nzpsi, iy, wy, wy, lo, hi, t, cy, cy);
-      __syncthreads();
+      lds_sync<kWave>();
       // the probe value of the next iteration is loaded one iteration ahead
       float2 pnext = prow[dct_nat<N>(t)];
 #pragma unroll 2
@@ -230,9 +231,9 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(4))
     // the transform's first stage reads only the slots t + e T this thread
     // wrote, so no ordering point is needed before it; the last stage writes
     // the row to T in natural order from registers
-    fresnel_1d<N, E, kMaxRadix, false, LineStore<N>>(
+    fresnel_1d<N, E, kMaxRadix, kWave, LineStore<N>>(
         s, t, twr, tab, LineStore<N>{valid ? a.T + (bj * a.nz + ty) * (int64_t)N : nullptr, t, T});
-    __syncthreads();  // the next angle's gather writes s
+    lds_sync<kWave>();  // the next angle's gather writes s
   }
 }
 
@@ -268,6 +269,7 @@ struct BhResidual {
 template <int N, int E, int C>
 __global__ __launch_bounds__(C*(N / E)) void bh_cols_k(BhArgs a, int tiles_per_field) {
   constexpr int T = N / E, NT = C * T, LS = col_stride<N, C>();
+  constexpr bool kWave = wave_private<N, E>();
   __shared__ float2 lds[2 * C * LS];
   __shared__ double red[NT / 64 > 0 ? NT / 64 : 1];
   const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -290,10 +292,11 @@ __global__ __launch_bounds__(C*(N / E)) void bh_cols_k(BhArgs a, int tiles_per_f
   const float sc = a.scales[b].x;
   float objf = 0.0f;
   const BhResidual<E> res{dv, sc, objf};
-  fresnel_1d_pp<N, E, kMaxRadix, false, BhResidual<E>>(s0, s, t, twr, a.taby + (int64_t)(j * 2 + 0) * 3 * (N / 2),
+  fresnel_1d_pp<N, E, kMaxRadix, kWave, BhResidual<E>>(s0, s, t, twr, a.taby + (int64_t)(j * 2 + 0) * 3 * (N / 2),
                                                        res);
   double obj = (double)objf;
-  fresnel_1d_pp<N, E>(s, s0, t, twr, a.taby + (int64_t)(j * 2 + 1) * 3 * (N / 2));
+  fresnel_1d_pp<N, E, kMaxRadix, kWave>(s, s0, t, twr, a.taby + (int64_t)(j * 2 + 1) * 3 * (N / 2));
+  if constexpr (kWave) __syncthreads();  // the store crosses columns
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
   col_tile_xfer<N, E, C, false>(lds, base, a.n, tid);
@@ -359,6 +362,7 @@ __device__ __forceinline__ int64_t group_start(const int* pidx, int64_t nang, in
 template <int N, int E, typename TO, bool STAGED, bool SPLIT>
 __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   constexpr int T = N / E, ROWS = kRowThreads / T;
+  constexpr bool kWave = wave_private<N, E>();  // a row's buffers are one wavefront's
   __shared__ float2 lds[ROWS * fft_buf<N>()];
   __shared__ float2 lacc[ROWS * N];  // probe-gradient accumulator of the row
   __shared__ float2 red[kRowThreads / 64];
@@ -436,7 +440,7 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
     // its first ordering point also orders the staged rows; the epilogue reads
     // back only this thread's outputs (elements t + e T), so the last stage
     // needs no closing ordering point
-    fresnel_1d_from<N, E, kMaxRadix, false, OwnOutputs>(h, s, t, twr, tab);
+    fresnel_1d_from<N, E, kMaxRadix, kWave, OwnOutputs>(h, s, t, twr, tab);
     const int p = a.pidx ? a.pidx[b] : 0;
     if (p != pcur) {
       flush(pcur);
@@ -468,7 +472,7 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
     }
     const float2 tot = row_sum2<T>(make_float2(s1, s2), red);
     if (valid && t0 == 0) a.part_r[bj * a.nz + ty] = tot;
-    __syncthreads();
+    lds_sync<kWave>();
   }
   flush(pcur);
 }

@@ -271,7 +271,9 @@ __device__ __forceinline__ void hcol_transform_pp(HColPipe<N, E, C>& pp, float2*
   pp.put();
   if (next) pp.fetch(next);
   __syncthreads();
-  fresnel_1d_pp<N, E, kMaxRadix, false, EPI>(lds + cc * LS, lds + C * LS + cc * LS, t, twr, tab, epi);
+  constexpr bool kWave = wave_private<N, E>();
+  fresnel_1d_pp<N, E, kMaxRadix, kWave, EPI>(lds + cc * LS, lds + C * LS + cc * LS, t, twr, tab, epi);
+  if constexpr (kWave) __syncthreads();  // the next field's tile crosses columns
 }
 
 // Consumers of the column transforms (output hooks, nothing stored).

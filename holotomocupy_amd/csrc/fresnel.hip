@@ -47,7 +47,7 @@ __global__ __launch_bounds__(kRowThreads) void fresnel_rows_k(const float2* in, 
 #pragma unroll
   for (int e = 0; e < E; ++e) h[e] = valid ? src[dct_nat<N>(t + e * T)] : make_float2(0.f, 0.f);
   // the last stage writes the row to out in natural order from registers
-  fresnel_1d_from<N, E, kMaxRadix, false, LineStore<N>>(
+  fresnel_1d_from<N, E, kMaxRadix, wave_private<N, E>(), LineStore<N>>(
       h, s, t, twr, tab, LineStore<N>{valid ? out + fb * out_stride + fy * N : nullptr, t, T});
 }
 
@@ -72,7 +72,9 @@ __global__ __launch_bounds__(C*(N / E)) void fresnel_cols_k(float2* data, int64_
   fft_load_twiddles<N, E>(twr, t, tw);
   col_tile_xfer<N, E, C, true>(lds, base, n, threadIdx.x);  // FFT slot q holds row dct_nat(q)
   __syncthreads();
-  fresnel_1d<N, E>(lds + cc * LS, t, twr, tab);
+  constexpr bool kWave = wave_private<N, E>();
+  fresnel_1d<N, E, kMaxRadix, kWave>(lds + cc * LS, t, twr, tab);
+  if constexpr (kWave) __syncthreads();  // the store crosses columns
   col_tile_xfer<N, E, C, false>(lds, base, n, threadIdx.x);
 }
 

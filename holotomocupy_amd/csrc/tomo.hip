@@ -103,8 +103,8 @@ __global__ __launch_bounds__(256) void tomo_rows_fwd_k(TomoArgs a, const TI* __r
     }
     s[fpad(p)] = v;
   }
-  __syncthreads();
-  fft_lds<N2, E, false>(s, t, twr);
+  lds_sync<wave_private<N2, E>()>();
+  fft_lds<N2, E, false, kMaxRadix, wave_private<N2, E>()>(s, t, twr);
   if (valid) {
     float2* dst = a.W + (z * n + ip) * (int64_t)N2;
 #pragma unroll
@@ -136,7 +136,8 @@ __global__ __launch_bounds__(C*(N2 / E)) void tomo_cols_fwd_k(TomoArgs a) {
     lds[c * LS + fpad(i)] = (i >= h && i < h + n) ? src[(i - h) * N2 + c] : make_float2(0.f, 0.f);
   }
   __syncthreads();
-  fft_lds<N2, E, false>(lds + cc * LS, t, twr);
+  fft_lds<N2, E, false, kMaxRadix, wave_private<N2, E>()>(lds + cc * LS, t, twr);
+  if constexpr (wave_private<N2, E>()) __syncthreads();  // the store crosses columns
   float2* dst = a.G + z * (int64_t)N2 * N2 + k0;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(C*(N / E)) void tomo_line_ifft_k(TomoArgs a, TO* __
   }
   __syncthreads();
   float2* s = lds + cc * LS;
-  fft_lds<N, E, true>(s, t, twr);
+  fft_lds<N, E, true, kMaxRadix, wave_private<N, E>()>(s, t, twr);
   if (l0 + cc < (int64_t)a.ntheta * a.nz) {
     TO* dst = out + (l0 + cc) * N;
 #pragma unroll
@@ -359,8 +360,9 @@ __global__ __launch_bounds__(C*(N / E)) void tomo_linefft_k(TomoArgs a, const TI
     const int tt = t + e * T;
     s[fpad(tt)] = valid ? cscale(ld_c<TI>(src, tt), -sgnf(tt)) : make_float2(0.f, 0.f);
   }
-  __syncthreads();
-  fft_lds<N, E, false>(s, t, twr);
+  lds_sync<wave_private<N, E>()>();
+  fft_lds<N, E, false, kMaxRadix, wave_private<N, E>()>(s, t, twr);
+  if constexpr (wave_private<N, E>()) __syncthreads();  // the store crosses lines
   const int c = threadIdx.x % C, p0 = threadIdx.x / C;
   if (l0 + c >= lines) return;
   const LineIdx li(a, l0 + c);
@@ -646,7 +648,8 @@ __global__ __launch_bounds__(C*(N2 / E)) void tomo_cols_adj_k(TomoArgs a) {
     lds[c * LS + fpad(k)] = cscale(src[k * N2 + c], sgnf(k + k0 + c));
   }
   __syncthreads();
-  fft_lds<N2, E, true>(lds + cc * LS, t, twr);
+  fft_lds<N2, E, true, kMaxRadix, wave_private<N2, E>()>(lds + cc * LS, t, twr);
+  if constexpr (wave_private<N2, E>()) __syncthreads();  // the store crosses columns
   float2* dst = a.W + z * (int64_t)n * N2 + k0;
   const float sc = 1.0f / N2;
 #pragma unroll
@@ -677,8 +680,8 @@ __global__ __launch_bounds__(256) void tomo_rows_adj_k(TomoArgs a, TO* __restric
     const int k = t + e * T;
     s[fpad(k)] = src[k];
   }
-  __syncthreads();
-  fft_lds<N2, E, true>(s, t, twr);
+  lds_sync<wave_private<N2, E>()>();
+  fft_lds<N2, E, true, kMaxRadix, wave_private<N2, E>()>(s, t, twr);
   if (valid) {
     TO* dst = out + (z * n + ip) * (int64_t)n;
     const float sc = 1.0f / N2;

@@ -222,16 +222,19 @@ def test_fused_gradient_bench_size_properties(gpu):
     assert rel(gs["prb"], g1["prb"].cpu().numpy()) < 1e-6
 
 
-@pytest.mark.parametrize("n,ndist,runs", [(64, 2, (1, 4, 5, 9, 3)), (128, 3, (70, 1, 8))])
-def test_probe_runs_alone_and_together(gpu, n, ndist, runs):
+@pytest.mark.parametrize("n,ndist,runs,real", [(64, 2, (1, 4, 5, 9, 3), False), (128, 3, (70, 1, 8), False),
+                                               (32, 1, (2, 5), True), (256, 2, (3, 5), False), (256, 1, (4, 2), True),
+                                               (512, 1, (1, 5), False), (512, 2, (2, 3), True),
+                                               (1024, 1, (2, 5), False), (1024, 1, (1, 4), True)])
+def test_probe_runs_alone_and_together(gpu, n, ndist, runs, real):
     """Groups of angles whose probe-gradient sums are formed apart and added:
     runs shorter than, equal to and longer than a group (and than the 64
     angles that one look back covers) give the same bits alone and in one
     launch, and the per-operator cascade's gradient."""
-    print(f"[case] probe runs n={n} ndist={ndist} runs={runs}", flush=True)
+    print(f"[case] probe runs n={n} ndist={ndist} runs={runs} real={real}", flush=True)
     from holotomocupy_amd.bh import BHGradient
     B = sum(runs)
-    rec, cas, x, v, w, d = make_problem(False, n=n, nobj=48, ndist=ndist, B=B, seed=61)
+    rec, cas, x, v, w, d = make_problem(real, n=n, nobj=48, ndist=ndist, B=B, seed=61)
     xd, dd = dev(x), torch.from_numpy(d).cuda()
     bh = BHGradient(rec)
     mag = rec.eff_demagnifications[:B].contiguous()

@@ -330,7 +330,10 @@ __global__ __launch_bounds__(C*(N / E)) void bh_cols_k(BhArgs a, int tiles_per_f
 // bh_prb_final_k adds the groups.  The groups are counted from the first angle
 // of the probe's run, and their size and the use of SPLIT depend on the
 // geometry alone, so the order of the sum, and with it every bit of a request's
-// result, does not depend on what else is in the batch.
+// result, does not depend on what else is in the batch.  maxgroups counts one
+// run to a probe; where an overwriting call has more, the last group takes all
+// angles that are left, for their object and position gradients (the probe
+// gradients of such a call are not defined).
 constexpr int kAdjGroup = 4;
 
 // First angle of group q (nang: there are not so many groups).  Every run of
@@ -359,6 +362,19 @@ __device__ __forceinline__ int64_t group_start(const int* pidx, int64_t nang, in
   return nang;
 }
 
+// One past the last angle of the group that starts at b.
+__device__ __forceinline__ int64_t group_end(const int* pidx, int64_t nang, int64_t b) {
+  if (!pidx) return min(b + kAdjGroup, nang);
+  int64_t e = b + 1;
+  bool same = true;
+#pragma unroll
+  for (int k = 1; k < kAdjGroup; ++k) {
+    same = same && b + k < nang && pidx[min(b + k, nang - 1)] == pidx[b];
+    e += same;
+  }
+  return e;
+}
+
 template <int N, int E, typename TO, bool STAGED, bool SPLIT>
 __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   constexpr int T = N / E, ROWS = kRowThreads / T;
@@ -376,7 +392,7 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   const int64_t unit = row_tile(blockIdx.x - q * ublocks, ublocks, a.ndist) * ROWS + r;
   const int64_t b0 = SPLIT ? group_start(a.pidx, a.nang, q) : 0;
   if (b0 >= a.nang) return;  // the whole workgroup
-  const int64_t b1 = SPLIT ? min(b0 + kAdjGroup, a.nang) : a.nang;
+  const int64_t b1 = SPLIT && q + 1 < a.maxgroups ? group_end(a.pidx, a.nang, b0) : a.nang;
   const bool valid = unit < nunits;
   const int j = valid ? (int)(unit / a.nz) : 0, ty = valid ? (int)(unit % a.nz) : 0;
   float2* s = lds + r * fft_buf<N>();
@@ -411,9 +427,6 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
     }
   };
   for (int64_t b = b0; b < b1; ++b) {
-    if constexpr (SPLIT) {
-      if (a.pidx && a.pidx[b] != pcur) break;  // the run ends inside the group
-    }
     int t = t0;
     asm volatile("" : "+v"(t));
     const int64_t bj = b * a.ndist + j;
@@ -442,7 +455,7 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
     // needs no closing ordering point
     fresnel_1d_from<N, E, kMaxRadix, kWave, OwnOutputs>(h, s, t, twr, tab);
     const int p = a.pidx ? a.pidx[b] : 0;
-    if (p != pcur) {
+    if (!SPLIT && p != pcur) {
       flush(pcur);
       pcur = p;
     }
@@ -573,14 +586,16 @@ __global__ __launch_bounds__(256) void bh_prb_final_k(BhArgs a) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= field) return;
   const float2* part = a.part_g + i;
-  for (int64_t first = 0; first < a.nang;) {
+  int64_t left = a.maxgroups;
+  for (int64_t first = 0; first < a.nang && left > 0;) {
     const int p = a.pidx ? a.pidx[first] : 0;
     int64_t end = a.nang;
     if (a.pidx)
       for (end = first + 1; end < a.nang && a.pidx[end] == p; ++end) {
       }
     float2 tot = make_float2(0.f, 0.f);
-    const int64_t groups = (end - first + kAdjGroup - 1) / kAdjGroup;
+    const int64_t groups = min((end - first + kAdjGroup - 1) / kAdjGroup, left);
+    left -= groups;
 #pragma unroll 4
     for (int64_t k = 0; k < groups; ++k) tot = cadd(tot, part[k * field]);
     part += groups * field;

@@ -276,3 +276,32 @@ def test_angles_split_over_workgroups_with_a_remainder(gpu):
     for z in (yd, dev(w)):
         h = rec.hessian_fused(xd, yd, yd if z is yd else z, dd).item()
         assert h == pytest.approx(rec.hessian_cascade(xd, yd, yd if z is yd else z, dd), rel=1e-4)
+
+
+def test_tab_call_with_scattered_probes(gpu):
+    """A batch by address table whose angles take their probes in turn: more
+    runs of equal probes than probes (only the probe gradients ask for one run
+    each).  Every angle's object and position gradient is that of the angle
+    alone, and no output is left from before."""
+    print("[case] address table, probes in turn", flush=True)
+    from holotomocupy_amd.bh import BHGradient
+    B, k = 13, 2
+    rec, cas, x, v, w, d = make_problem(False, n=64, nobj=48, ndist=2, B=B, seed=63)
+    bh = BHGradient(rec)
+    xd, dd = dev(x), torch.from_numpy(d).cuda()
+    prb = [xd["prb"].clone(), xd["prb"] * (0.8 + 0.1j)]
+    gprb = [torch.empty_like(p) for p in prb]
+    gproj, gpos = torch.full_like(xd["proj"], float("nan")), torch.full_like(xd["pos"], float("nan"))
+    pidx = torch.arange(B, dtype=torch.int32, device="cuda") % k
+    mag = rec.eff_demagnifications[:B].contiguous()
+    s, rp = bh.scales(B)
+    tab = torch.tensor([t[b].data_ptr() for t in (xd["proj"], dd, gproj) for b in range(B)]
+                       + [t.data_ptr() for t in prb + gprb], dtype=torch.int64, device="cuda")
+    ws = torch.full((bh.workspace_bytes(B),), 0xff, dtype=torch.uint8, device="cuda")
+    bh.call_tab(tab, B, k, xd["pos"], mag, pidx, s, rp.repeat(k), gpos, ws)
+    for b in range(B):
+        one = {"prb": torch.zeros_like(prb[0]), "proj": torch.empty_like(gproj[b:b + 1]),
+               "pos": torch.empty_like(gpos[b:b + 1])}
+        rec.gradients_fused({"prb": prb[b % k], "proj": xd["proj"][b:b + 1], "pos": xd["pos"][b:b + 1]}, one,
+                            dd[b:b + 1], st=b)
+        assert torch.equal(one["proj"][0], gproj[b]) and torch.equal(one["pos"][0], gpos[b]), b

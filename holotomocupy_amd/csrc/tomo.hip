@@ -62,7 +62,7 @@ struct TomoArgs {
   float2* Sh = nullptr;            // [ntheta n, nz] line spectra, slices fastest
   const int* heavy = nullptr;      // tiles with more than kHeavyTile entries, longest first
   int nheavy = 0;
-  int longest = 0;                 // entries of the longest list
+  int parts = 0;                   // sums that a heavy list is cut into (4 or 16)
   // per-bin factor of the adjoint's line transform (NULL = none): the
   // detector filter of filtered back-projection, shifted by n/2 to the bins
   // of the c1d-modulated transform and scaled by sqrt(n / ntheta)
@@ -426,25 +426,32 @@ __global__ __launch_bounds__(256) void tomo_filter_k(const TIO* in, TIO* out, in
 // separate products, so 2 VEC U accumulators) and forms the weight of point
 // l % 16 from the sample's two zero-padded weight rows (built in FP64).  The
 // order of each sum is the list's, whatever runs when; no atomics.
-// The four wavefronts of a workgroup take four tiles of a row, which share most
-// of their samples and make whole cache lines of the result.  Every line crosses the centre, so the lists there are long (2500
-// samples at 256^2, 384 angles, against a mean of 54): the tiles with more
-// than kHeavyTile entries (listed longest first, at the front of the launch)
-// take a whole workgroup, which cuts the list in four and adds the four sums
-// in order.
+// The NW wavefronts of a workgroup take NW tiles of a row, which share most
+// of their samples and make whole cache lines of the result.  Every line crosses
+// the centre, so the lists there are long (2500 samples at 256^2, 384 angles,
+// against a mean of 54): the tiles with more than kHeavyTile entries (listed
+// longest first, at the front of the launch) take a whole workgroup each.  The
+// plan cuts these lists into parts, 16 where the longest has more than kLongTile
+// entries and else 4, whose sums are added four by four and the quarters in
+// order; a wavefront takes SUBS parts, and with four of them adds a quarter
+// itself.  So the order of a sum, and with it every bit of a slice's result, does
+// not depend on the slab that the slice comes in.
 // 256 slices of 256^2, 384 angles: 1555 us with a sum per point -> 390 us (1.2 GB
 // through the L2 misses, a third of it the grid; the products themselves are 104 us);
 // 45 real slices of 512^2, 451 angles (filtered back-projection): 1645 -> 275 us.
 constexpr int kHeavyTile = 128;
 constexpr int kLongTile = 512;  // from here more wavefronts share a long list (few slices)
+constexpr int kParts = 16, kQuarters = 4;
 constexpr int kBatch = 4;  // steps of four samples taken together
 
-template <int VEC, int U, int NW>
+template <int VEC, int U, int NW, int SUBS>
 __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
   constexpr int NA = 2 * VEC * U;  // accumulators: float columns of 16 slices
   constexpr int PX = 4 * NW;       // points of a workgroup's row
   constexpr int ZS = 4 * PX + 2;   // float2 slots of a slice's 4 rows, padded off its bank
-  constexpr int kOut = 16 * VEC * U * ZS / 2, kPart = (NW - 1) * NA * 64;
+  constexpr int SL = NW == kQuarters ? kQuarters : kParts;  // sums that the wavefronts hand over
+  static_assert(SL == (SUBS == 4 ? NW : NW * SUBS), "a quarter or a part in each slot");
+  constexpr int kOut = 16 * VEC * U * ZS / 2, kPart = SL * NA * 64;
   __shared__ f32x4 lds[kOut > kPart ? kOut : kPart];
   __shared__ int skipped[NW];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
@@ -452,12 +459,20 @@ __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
   const int nt = a.n / 2, n2 = 2 * a.n;
   const bool heavy = (int)blockIdx.x < a.nheavy;
   bool skip = false;  // nothing of this wavefront's is stored
-  int tile, beg, end;
+  int tile, beg, end, stop = 0;  // stop: where the part in hand ends (SUBS > 1)
+  // part i of a heavy list begins here: whole batches to a part
+  int first = 0, last = 0;
+  auto part_at = [&](int i) {
+    constexpr int B = 4 * kBatch;
+    return min(first + (int)((int64_t)((last - first + B - 1) / B) * i / (NW * SUBS)) * B, last);
+  };
   if (heavy) {
     tile = a.heavy[blockIdx.x];
-    const int b = a.tp[tile], steps = (a.tp[tile + 1] - b) / 4;
-    beg = b + steps * wv / NW * 4;
-    end = b + steps * (wv + 1) / NW * 4;
+    first = a.tp[tile];
+    last = a.tp[tile + 1];
+    beg = part_at(wv * SUBS);
+    end = part_at((wv + 1) * SUBS);
+    stop = part_at(wv * SUBS + 1);
   } else {
     const int nb = (nt + NW - 1) / NW;
     const int bid = (int)xcd_tile(blockIdx.x - a.nheavy, gridDim.x - a.nheavy);
@@ -467,6 +482,7 @@ __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
     end = a.tp[tile + 1];
     skip = tx >= nt || end - beg > kHeavyTile;
     if (skip) end = beg;
+    if constexpr (SUBS > 1) stop = end;
   }
   const int z0 = blockIdx.y * zper, z1 = min(z0 + zper, a.nz);
   int zc[U];
@@ -522,6 +538,29 @@ __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
 #pragma unroll
     for (int i = 0; i < NA; ++i) tot[i] += acc[i];
   };
+  // a wavefront of several parts keeps the sum of those before the one in hand
+  // in the lane's own slot (of four parts all, of two the first)
+  f32x4(*slot)[NA][64] = reinterpret_cast<f32x4(*)[NA][64]>(lds);
+  const int own = wv * SL / NW;
+  int sub = wv * SUBS + 1;
+  auto cut = [&](int e) {  // e: one past the last entry taken
+    if constexpr (SUBS > 1) {
+      if (__builtin_expect(e < stop || stop >= end, 1)) return;
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        slot[own][i][lane] = SUBS == 2 ? tot[i] : slot[own][i][lane] + tot[i];
+        tot[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      while (stop <= e && stop < end) stop = part_at(++sub);
+    }
+  };
+  if constexpr (SUBS > 1) {
+    if (heavy) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) slot[own][i][lane] = f32x4{0.f, 0.f, 0.f, 0.f};
+      while (stop <= beg && stop < end) stop = part_at(++sub);
+    }
+  }
   if (beg < end) {
     float w0[kBatch], v0[kBatch][U][2 * VEC];
     entries(beg);
@@ -537,42 +576,63 @@ __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
         if (more1) load(e + 4 * kBatch, w1, v1);
         mul(w0, v0);
         if (!more1) break;
+        cut(e + 4 * kBatch);
         if (more2) load(e + 8 * kBatch, w0, v0);
         mul(w1, v1);
         if (!more2) break;
+        cut(e + 8 * kBatch);
       }
     } else {
 #pragma unroll 1
       for (int e = beg; e < end; e += 4 * kBatch) {
         load(e, w0, v0);
         mul(w0, v0);
+        cut(e + 4 * kBatch);
       }
     }
   }
   const int64_t plane = (int64_t)n2 * n2;
   if (heavy) {
-    f32x4(*part)[NA][64] = reinterpret_cast<f32x4(*)[NA][64]>(lds);
-    if (wv) {
+    auto put = [&](int u, int c, f32x4 re, f32x4 im) {
+      const int zs = z0 + (u * 16 + q) * VEC;
+      if (zs >= z1) return;
+      float2* d = a.G + (int64_t)(tile / nt * 4 + kk) * n2 + tile % nt * 4 + (min(zs, a.nz - VEC) + c) * plane;
+      *reinterpret_cast<f32x4u*>(d) = f32x4{re.x, im.x, re.y, im.y};
+      *reinterpret_cast<f32x4u*>(d + 2) = f32x4{re.z, im.z, re.w, im.w};
+    };
+    if constexpr (SUBS == 4) {
 #pragma unroll
-      for (int i = 0; i < NA; ++i) part[wv - 1][i][lane] = tot[i];
+      for (int i = 0; i < NA; ++i) tot[i] = slot[own][i][lane] + tot[i];
+    }
+    if (SL == kParts || wv) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) slot[own + (SUBS == 2)][i][lane] = tot[i];
     }
     __syncthreads();
-    if (wv) return;
+    if constexpr (SL == kParts) {  // wavefront w the columns of slices (u, c) = w
+      if (wv >= U * VEC) return;
+      f32x4 sum[2];
 #pragma unroll
-    for (int k = 0; k < NW - 1; ++k)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int i = 0; i < NA; ++i) tot[i] += part[k][i][lane];
-    float2* dst = a.G + (int64_t)(tile / nt * 4 + kk) * n2 + tile % nt * 4;
+        for (int k = 0; k < SL; k += 4) {
+          f32x4 quarter = slot[k][2 * wv + i][lane];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+          for (int l = 1; l < 4; ++l) quarter += slot[k + l][2 * wv + i][lane];
+          sum[i] = k ? sum[i] + quarter : quarter;
+        }
+      put(wv / VEC, wv % VEC, sum[0], sum[1]);
+    } else {
+      if (wv) return;
 #pragma unroll
-      for (int c = 0; c < VEC; ++c) {
-        if (z0 + (u * 16 + q) * VEC >= z1) continue;
-        const f32x4 re = tot[(u * VEC + c) * 2], im = tot[(u * VEC + c) * 2 + 1];
-        float2* d = dst + (zc[u] + c) * plane;
-        *reinterpret_cast<f32x4u*>(d) = f32x4{re.x, im.x, re.y, im.y};
-        *reinterpret_cast<f32x4u*>(d + 2) = f32x4{re.z, im.z, re.w, im.w};
-      }
+      for (int k = 1; k < SL; ++k)
+#pragma unroll
+        for (int i = 0; i < NA; ++i) tot[i] += slot[k][i][lane];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) put(u, c, tot[(u * VEC + c) * 2], tot[(u * VEC + c) * 2 + 1]);
+    }
     return;
   }
   // result rows 4 (l / 16) + r are the points (y = l / 16, x = r), columns q
@@ -612,18 +672,26 @@ static hipError_t launch_grid_gather(const TomoArgs& a, hipStream_t st) {
   const int nt = a.n / 2;
   const int zblocks = (a.nz + 63) / 64, zper = ((a.nz + zblocks - 1) / zblocks + 1) / 2 * 2;
   auto grid = [&](int nw) { return dim3((unsigned)(a.nheavy + (nt + nw - 1) / nw * nt), (unsigned)zblocks); };
-  if (zper <= 16 && a.longest > kLongTile)
-    hipLaunchKernelGGL((tomo_grid_k<1, 1, 16>), grid(16), dim3(1024), 0, st, a, zper);
+#define HTAMD_GRID(VEC, U, NW, SUBS) \
+  hipLaunchKernelGGL((tomo_grid_k<VEC, U, NW, SUBS>), grid(NW), dim3(64 * NW), 0, st, a, zper)
+  const bool parts = a.parts == kParts;
+  if (zper <= 16 && parts)
+    HTAMD_GRID(1, 1, 16, 1);
   else if (zper <= 16)
-    hipLaunchKernelGGL((tomo_grid_k<1, 1, 4>), grid(4), dim3(256), 0, st, a, zper);
-  else if (zper <= 32 && a.longest > kLongTile)
-    hipLaunchKernelGGL((tomo_grid_k<2, 1, 8>), grid(8), dim3(512), 0, st, a, zper);
+    HTAMD_GRID(1, 1, 4, 1);
+  else if (zper <= 32 && parts)
+    HTAMD_GRID(2, 1, 8, 2);
   else if (zper <= 32)
-    hipLaunchKernelGGL((tomo_grid_k<2, 1, 4>), grid(4), dim3(256), 0, st, a, zper);
+    HTAMD_GRID(2, 1, 4, 1);
+  else if (zper <= 48 && parts)
+    HTAMD_GRID(1, 3, 4, 4);
   else if (zper <= 48)
-    hipLaunchKernelGGL((tomo_grid_k<1, 3, 4>), grid(4), dim3(256), 0, st, a, zper);
+    HTAMD_GRID(1, 3, 4, 1);
+  else if (parts)
+    HTAMD_GRID(2, 2, 4, 4);
   else
-    hipLaunchKernelGGL((tomo_grid_k<2, 2, 4>), grid(4), dim3(256), 0, st, a, zper);
+    HTAMD_GRID(2, 2, 4, 1);
+#undef HTAMD_GRID
   return hipGetLastError();
 }
 
@@ -969,7 +1037,7 @@ struct htamd_tomo_plan {
   int2* ge = nullptr;
   int* gc = nullptr;
   int* heavy = nullptr;
-  int nitems = 0, nheavy = 0, longest = 0, sparse = 0;
+  int nitems = 0, nheavy = 0, parts = 0, sparse = 0;
   // detector filters (ramp, Shepp-Logan, Parzen): [3][n] with the 1/n of the
   // inverse transform for htamd_tomo_filter, and [3][n] shifted by n/2 and
   // scaled by sqrt(n / ntheta) for htamd_tomo_fbp
@@ -1139,7 +1207,7 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
         make_int2((int)si, wrap(tb[(size_t)si].y) % kRG % py << 8 | wrap(tb[(size_t)si].x) % kRG % px);
   p->nitems = (int)items.size();
   p->nheavy = (int)heavy.size();
-  p->longest = heavy.empty() ? 0 : tp[(size_t)heavy[0] + 1] - tp[(size_t)heavy[0]];
+  p->parts = !heavy.empty() && tp[(size_t)heavy[0] + 1] - tp[(size_t)heavy[0]] > kLongTile ? kParts : kQuarters;
   // deapodiser phi (tomo.py:19-21, 46-47) with the mask folded in
   std::vector<float> phi((size_t)(n * n));
   for (int64_t i = 0; i < n; ++i) {
@@ -1241,7 +1309,7 @@ static int tomo_run(const htamd_tomo_plan* p, bool adjoint, const void* in, int 
   a.sparse = p->sparse;
   a.heavy = p->heavy;
   a.nheavy = p->nheavy;
-  a.longest = p->longest;
+  a.parts = p->parts;
   a.W = (float2*)ws;
   a.G = (float2*)ws + nz * p->n * 2 * p->n;
   a.Sh = a.G + nz * 4 * p->n * p->n;

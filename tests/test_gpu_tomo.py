@@ -256,3 +256,23 @@ def test_slab_sizes_at_the_edges_of_the_slice_blocks(gpu, n, ntheta, nz):
     for k in range(nz):
         assert rel(y[:, k], yo[:, k]) < REL_TOL, k
         assert rel(z[k], zo[k]) < REL_TOL, k
+
+
+@pytest.mark.parametrize("n,ntheta", [(64, 96), (64, 24), (50, 131)])
+def test_slices_keep_their_bits_in_any_slab(gpu, n, ntheta):
+    """R, RT and fbp of a slice do not depend on the slab that it comes in: the
+    slab sizes on either side of every choice of launch, with central lists of
+    over 512 samples (664 and 892) and shorter ones."""
+    from holotomocupy_amd import Tomo
+    print(f"[case] slices in slabs n={n} ntheta={ntheta}", flush=True)
+    rng = np.random.default_rng(n)
+    nz = 65
+    t = Tomo(n, nz, angles(ntheta), 0)
+    x, d = dev(data(rng, (nz, n, n), False)), dev(data(rng, (ntheta, nz, n), False))
+    full = t.R(x), t.RT(d), t.fbp(d)
+    for k in (1, 2, 8, 9, 16, 17, 24, 32, 33, 40, 48, 49, 64):
+        z0 = (nz - k) // 2  # an odd start as well as an even one
+        y, s = x[z0:z0 + k].contiguous(), d[:, z0:z0 + k].contiguous()
+        assert torch.equal(t.R(y), full[0][:, z0:z0 + k]), k
+        assert torch.equal(t.RT(s), full[1][z0:z0 + k]), k
+        assert torch.equal(t.fbp(s), full[2][z0:z0 + k]), k

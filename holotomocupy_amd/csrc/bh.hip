@@ -41,9 +41,12 @@ struct BhArgs {
   int accumulate_prb = 0;
   float2* part_r = nullptr;          // [nang*ndist*nz] shift-gradient partials
   double* part_obj = nullptr;        // [column tiles] objective partials
-  float2* part_g = nullptr;          // split angles: [groups <= nang, ndist, nz, n] probe-gradient sums of the
-                                     // groups (NULL: not split)
+  float2* part_g = nullptr;          // split angles: [slots, ndist, nz, n] probe-gradient sums of the groups of
+                                     // one window (NULL: not split)
   int64_t maxgroups = 0;             // no more groups than this
+  int64_t window = 0;                // groups that part_g holds; where there may be more, the slot after them
+                                     // carries the sum of a run from one window into the next
+  int64_t group0 = 0, ngroups = 0;   // the window in hand: first group, groups
   int64_t groups = 1;                // groups of angles of K1
   const float2* twx = nullptr;
   const float2* twy = nullptr;
@@ -388,8 +391,8 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   // are the last ones of the launch (dispatched among the others they would
   // leave the same shader engines idle each time)
   const int64_t ublocks = (nunits + ROWS - 1) / ROWS;
-  const int64_t q = SPLIT ? blockIdx.x / ublocks : 0;
-  const int64_t unit = row_tile(blockIdx.x - q * ublocks, ublocks, a.ndist) * ROWS + r;
+  const int64_t slot = SPLIT ? blockIdx.x / ublocks : 0, q = a.group0 + slot;
+  const int64_t unit = row_tile(blockIdx.x - slot * ublocks, ublocks, a.ndist) * ROWS + r;
   const int64_t b0 = SPLIT ? group_start(a.pidx, a.nang, q) : 0;
   if (b0 >= a.nang) return;  // the whole workgroup
   const int64_t b1 = SPLIT && q + 1 < a.maxgroups ? group_end(a.pidx, a.nang, b0) : a.nang;
@@ -408,7 +411,7 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
   auto flush = [&](int p) {
     if (!valid) return;
     if constexpr (SPLIT) {
-      float2* g = a.part_g + ((q * a.ndist + j) * a.nz + ty) * (int64_t)N;
+      float2* g = a.part_g + ((slot * a.ndist + j) * a.nz + ty) * (int64_t)N;
       for (int e = 0; e < E; ++e) {
         const int i = dct_nat<N>(t0 + e * T);
         g[i] = acc[i];
@@ -580,28 +583,36 @@ __global__ __launch_bounds__(256) void bh_pos_final_k(const float2* __restrict__
 }
 
 // Probe gradients of the split K3: per element the group sums of each run of
-// angles in order, then times rho_prb^2 into (or onto) the run's probe.
+// angles in order, then times rho_prb^2 into (or onto) the run's probe.  One
+// window of groups; a run that it does not finish goes on in the next.
 __global__ __launch_bounds__(256) void bh_prb_final_k(BhArgs a) {
   const int64_t field = (int64_t)a.ndist * a.nz * a.n;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= field) return;
   const float2* part = a.part_g + i;
-  int64_t left = a.maxgroups;
-  for (int64_t first = 0; first < a.nang && left > 0;) {
+  float2* carry = a.part_g + a.window * field + i;
+  const int64_t stop = a.group0 + a.ngroups;
+  int64_t q = 0;  // first group of the run
+  for (int64_t first = 0; first < a.nang && q < stop;) {
     const int p = a.pidx ? a.pidx[first] : 0;
     int64_t end = a.nang;
     if (a.pidx)
       for (end = first + 1; end < a.nang && a.pidx[end] == p; ++end) {
       }
-    float2 tot = make_float2(0.f, 0.f);
-    const int64_t groups = min((end - first + kAdjGroup - 1) / kAdjGroup, left);
-    left -= groups;
+    const int64_t qend = q + (end - first + kAdjGroup - 1) / kAdjGroup, k1 = min(qend, stop);
+    if (qend > a.group0) {
+      float2 tot = q < a.group0 ? *carry : make_float2(0.f, 0.f);
 #pragma unroll 4
-    for (int64_t k = 0; k < groups; ++k) tot = cadd(tot, part[k * field]);
-    part += groups * field;
-    float2* g = (a.gprb_p ? a.gprb_p[p] : a.gprb + p * field) + i;
-    const float2 v = cscale(tot, a.rho_prb[p]);
-    *g = a.accumulate_prb ? cadd(*g, v) : v;
+      for (int64_t k = max(q, a.group0); k < k1; ++k) tot = cadd(tot, part[(k - a.group0) * field]);
+      if (k1 == qend || stop == a.maxgroups) {
+        float2* g = (a.gprb_p ? a.gprb_p[p] : a.gprb + p * field) + i;
+        const float2 v = cscale(tot, a.rho_prb[p]);
+        *g = a.accumulate_prb ? cadd(*g, v) : v;
+      } else {
+        *carry = tot;
+      }
+    }
+    q = qend;
     first = end;
   }
 }
@@ -624,6 +635,7 @@ __global__ __launch_bounds__(256) void bh_sum_k(const double* __restrict__ part,
 
 struct BhLayout {
   int64_t c = 0, T = 0, dpsi = 0, part_r = 0, part_obj = 0, part_g = 0, total = 0;
+  int64_t slots = 0;  // of part_g (0: K3 does not split the angles)
 };
 
 // Column pass of the fused gradient: 16 elements per thread at N = 2048 (two
@@ -709,6 +721,14 @@ static bool adj_split(int64_t n, int64_t nz, int64_t ndist, int64_t npsi, int64_
 // split 1979 -> 2002 us).
 constexpr int64_t kFwdBlocks = 4096;
 
+// Slots of the group sums.  One run of angles has a quarter as many groups as
+// angles, runs of five angles 2/5, and only shorter ones more: such calls take
+// several windows.  Up to eight slots, and as many as the object gradient has
+// room for (it is formed after the group sums have been used), cost nothing.
+static int64_t adj_slots(int64_t nang, int64_t slot_bytes, int64_t dpsi_bytes) {
+  return std::min(nang, std::max({(int64_t)8, (2 * nang + 4) / 5, dpsi_bytes / slot_bytes}));
+}
+
 static BhLayout bh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* sp, int64_t nang) {
   BhLayout L;
   const int64_t osz = sp->is_complex ? 8 : 4;
@@ -721,13 +741,18 @@ static BhLayout bh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* sp,
   L.T = off;
   off += align256(nang * pp->ndist * field * 8);
   L.dpsi = off;
-  off += align256(nang * plane * osz);
+  L.part_g = off;
+  int64_t room = nang * plane * osz;
+  if (nang > kAdjGroup && adj_split(pp->n, pp->nz, pp->ndist, sp->npsi, osz)) {  // up to one group: the same sum either way
+    const int64_t slot = pp->ndist * field * 8;
+    L.slots = adj_slots(nang, slot, room);
+    room = std::max(room, L.slots * slot);
+  }
+  off += align256(room);
   L.part_r = off;
   off += align256(nang * pp->ndist * pp->nz * 8);
   L.part_obj = off;
   off += align256(ntiles * 8);
-  L.part_g = off;
-  if (nang > kAdjGroup && adj_split(pp->n, pp->nz, pp->ndist, sp->npsi, osz)) off += align256(nang * pp->ndist * field * 8);
   L.total = off;
   return L;
 }
@@ -747,23 +772,29 @@ static hipError_t launch_rows(bool adjoint, BhArgs a, hipStream_t st) {
   const int64_t dyn = rs.dyn;
   const bool staged = rs.staged, split = a.part_g != nullptr;
   a.groups = whole_rounds(rs.blocks, 4, rs.lds, 1) ? 1 : std::min(a.nang, (kFwdBlocks + rs.blocks - 1) / rs.blocks);
-  const int64_t grid = rs.blocks * (!adjoint ? a.groups : split ? a.maxgroups : 1);
-  if (adjoint) {
-    if (staged && split)
-      hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, true, true>), dim3((unsigned)grid), dim3(kRowThreads),
-                         (size_t)dyn, st, a);
-    else if (staged)
+  int64_t grid = rs.blocks * (adjoint ? 1 : a.groups);
+  if (adjoint && split) {
+    const int64_t field = units * N;
+    for (a.group0 = 0; a.group0 < a.maxgroups; a.group0 += a.ngroups) {
+      a.ngroups = std::min(a.window, a.maxgroups - a.group0);
+      grid = rs.blocks * a.ngroups;
+      if (staged)
+        hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, true, true>), dim3((unsigned)grid), dim3(kRowThreads),
+                           (size_t)dyn, st, a);
+      else
+        hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, false, true>), dim3((unsigned)grid), dim3(kRowThreads), 0, st,
+                           a);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(bh_prb_final_k, dim3((unsigned)((field + 255) / 256)), dim3(256), 0, st, a);
+    }
+  } else if (adjoint) {
+    if (staged)
       hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, true, false>), dim3((unsigned)grid), dim3(kRowThreads),
                          (size_t)dyn, st, a);
-    else if (split)
-      hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, false, true>), dim3((unsigned)grid), dim3(kRowThreads), 0, st, a);
     else
       hipLaunchKernelGGL((bh_adj_rows_k<N, E, TO, false, false>), dim3((unsigned)grid), dim3(kRowThreads), 0, st,
                          a);
-    if (split) {
-      const int64_t field = units * N;
-      hipLaunchKernelGGL(bh_prb_final_k, dim3((unsigned)((field + 255) / 256)), dim3(256), 0, st, a);
-    }
   } else {
     if (staged)
       hipLaunchKernelGGL((bh_fwd_rows_k<N, E, TO, true>), dim3((unsigned)grid), dim3(kRowThreads), (size_t)dyn,
@@ -973,11 +1004,12 @@ static int bh_gradient_impl(const htamd_bh_plan* p, int64_t nangles, const void*
   a.accumulate_prb = accumulate_prb;
   a.part_r = (float2*)(ws + L.part_r);
   a.part_obj = (double*)(ws + L.part_obj);
-  if (nangles > kAdjGroup && adj_split(a.n, a.nz, a.ndist, a.npsi, p->shift->is_complex ? 8 : 4)) {  // up to one group: the same sum either way
+  if (L.slots) {
     a.part_g = (float2*)(ws + L.part_g);
     // a run ends at most one group early; nprobes is not known without the table
     const int64_t full = (nangles + kAdjGroup - 1) / kAdjGroup;
     a.maxgroups = !probe_index ? full : tab && !accumulate_prb ? std::min(nangles, full + nprobes - 1) : nangles;
+    a.window = a.maxgroups <= L.slots ? a.maxgroups : L.slots - 1;
   }
   a.twx = p->prop->tw_x;
   a.twy = p->prop->tw_y;

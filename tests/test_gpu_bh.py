@@ -305,3 +305,55 @@ def test_tab_call_with_scattered_probes(gpu):
         rec.gradients_fused({"prb": prb[b % k], "proj": xd["proj"][b:b + 1], "pos": xd["pos"][b:b + 1]}, one,
                             dd[b:b + 1], st=b)
         assert torch.equal(one["proj"][0], gproj[b]) and torch.equal(one["pos"][0], gpos[b]), b
+
+
+@pytest.mark.parametrize("n,nobj,ndist,B", [(256, 256, 2, 48), (256, 128, 2, 48), (128, 128, 3, 9), (64, 48, 2, 300)])
+def test_gradient_workspace_holds_no_second_work_field(gpu, n, nobj, ndist, B):
+    """The group sums of the split row pass take the room of the object gradient,
+    which is formed after them, and beyond it at most two slots to five angles
+    (at least eight) where the work field has one per angle."""
+    print(f"[case] gradient workspace n={n} nobj={nobj} ndist={ndist} B={B}", flush=True)
+    from holotomocupy_amd.bh import BHGradient
+    rec = make_problem(False, n=n, nobj=nobj, ndist=ndist, B=1, seed=64)[0]
+    obj, slot = B * nobj * nobj * 8, ndist * n * n * 8
+    base = 2 * obj + B * slot + B * ndist * n * 16  # coefficients, object gradient, work field, partial sums
+    groups = min(B, max(8, -(-2 * B // 5)))
+    assert BHGradient(rec).workspace_bytes(B) <= base + max(0, groups * slot - obj) + 8 * 256
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_probe_runs_over_several_windows(gpu, accumulate):
+    """More groups of angles than their sums have slots (18 of 43 angles, 21
+    groups): a run that begins in one window of groups and ends in the next, and
+    runs of one angle on both sides, give the bits of each run alone."""
+    print(f"[case] probe runs over windows accumulate={accumulate}", flush=True)
+    from holotomocupy_amd.bh import BHGradient
+    runs = (1,) * 10 + (30,) + (1,) * 3
+    B, k = sum(runs), len(runs)
+    rec, cas, x, v, w, d = make_problem(False, n=64, nobj=32, ndist=2, B=B, seed=65)
+    xd, dd = dev(x), torch.from_numpy(d).cuda()
+    bh = BHGradient(rec)
+    mag = rec.eff_demagnifications[:B].contiguous()
+    prb = torch.stack([xd["prb"] * (1 + 0.1 * i) for i in range(k)]).contiguous()
+    pidx = torch.tensor(sum(([i] * m for i, m in enumerate(runs)), []), dtype=torch.int32, device="cuda")
+    s, rp = bh.scales(B)
+    before = 0.01 * prb.flip(0)
+    gproj, gpos, gprb = torch.empty_like(xd["proj"]), torch.empty_like(xd["pos"]), before.clone()
+    bh(prb, xd["proj"], xd["pos"], dd, mag, gproj, gpos, gprb, accumulate_prb=accumulate, probe_index=pidx, scales=s,
+       rho_prb=rp.repeat(k))
+    tprb = torch.empty_like(prb) if not accumulate else before.clone()
+    tproj, tpos = torch.empty_like(gproj), torch.empty_like(gpos)
+    tab = torch.tensor([t[b].data_ptr() for t in (xd["proj"], dd, tproj) for b in range(B)]
+                       + [t[i].data_ptr() for t in (prb, tprb) for i in range(k)], dtype=torch.int64, device="cuda")
+    ws = torch.full((bh.workspace_bytes(B),), 0xff, dtype=torch.uint8, device="cuda")
+    bh.call_tab(tab, B, k, xd["pos"], mag, pidx, s, rp.repeat(k), tpos, ws, accumulate_prb=accumulate)
+    assert torch.equal(tproj, gproj) and torch.equal(tpos, gpos) and torch.equal(tprb, gprb)
+    st = 0
+    for i, m in enumerate(runs):
+        sl = slice(st, st + m)
+        one = {"prb": before[i].clone() if accumulate else torch.zeros_like(prb[i]),
+               "proj": torch.empty_like(gproj[sl]), "pos": torch.empty_like(gpos[sl])}
+        rec.gradients_fused({"prb": prb[i], "proj": xd["proj"][sl], "pos": xd["pos"][sl]}, one, dd[sl], st=st)
+        assert torch.equal(one["prb"], gprb[i]), i
+        assert torch.equal(one["proj"], gproj[sl]) and torch.equal(one["pos"], gpos[sl]), i
+        st += m

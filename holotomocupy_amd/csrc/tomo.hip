@@ -158,22 +158,27 @@ __global__ __launch_bounds__(C*(N2 / E)) void tomo_cols_fwd_k(TomoArgs a) {
 // cell holds about 8 samples at 256^2, 384 angles: 4x4 cells take a third more
 // products, 8x8 cells as many more at that density (fewer at sparser ones).
 // A workgroup stages a region of kRG x kRG first taps with the margin of the
-// windows, wrapped on the 2n grid, for 16 slices (slices fastest, a point's
-// row padded to 17: the lanes of a read are 16 slices of 4 neighbouring
+// windows, wrapped on the 2n grid, for Z slices (slices fastest, a point's
+// row padded to Z + 1: the lanes of a read are the slices of 4 neighbouring
 // points, the lanes of a staging write 12 pairs of points of one slice), and
 // its wavefronts take the groups in turn.
+// The 16 rows of a product are 16 slices (re and im in two products), 8 slices
+// x (re, im), or 4 slices x (re, im) x two patch rows; a sample's sum runs in the
+// same order in all three, and few slices pay neither for staging nor for
+// products of slices that are not there (one slice of 512^2, 451 angles: R takes
+// 99 us in sixteens, 47 us in fours; 8 slices of 512^2, 128 angles 102 and 74).
 // Each sample's two weight rows are read once per group; lane l holds sample
 // l % 16 and the points 4 j + l / 16 of a row.
 // Few angles leave a cell one or two samples: then a group is 16 samples of a
 // region (SPARSE), a workgroup takes one group, and its wavefronts share the
-// rows of the region's patch.  The plan takes the form of fewer steps (R at 8
-// slices of 512^2, 64 angles: 111 us with cells, 92 with regions; 100 slices of
-// 256^2, 100 angles: 272 and 316).
+// rows of the region's patch.  The plan takes the form of fewer steps, whatever
+// the slab, so that slices keep their bits (in sixteens, R at 8 slices of 512^2,
+// 64 angles: 111 us with cells, 92 with regions; 100 slices of 256^2, 100
+// angles: 272 and 316).
 // 256 slices of 256^2, 384 angles: 974 us with a thread per sample and four
 // slices -> 450 us (the products are 177 us).
 constexpr int kTL = 9;                        // taps along an axis
 constexpr int kRG = 16, kRP = kRG + kTL - 1;  // region and its staged edge
-constexpr int kRZ = 16, kRZP = kRZ + 1;       // slices, and the pitch of a staged point
 constexpr int kCellY = 4, kCellX = 8;
 constexpr int kItemGroups = 16;               // groups of a work item
 constexpr int kGatherWaves = 8;
@@ -188,11 +193,16 @@ struct GatherShape {
   static constexpr int NR = SPARSE ? kRP / kGatherWaves : NY;                // rows of a wavefront
 };
 
-template <bool SPARSE>
-__global__ __launch_bounds__(64 * kGatherWaves) __attribute__((amdgpu_waves_per_eu(4))) void tomo_gather_k(
+template <bool SPARSE, int Z>
+__global__ __launch_bounds__(64 * kGatherWaves) __attribute__((amdgpu_waves_per_eu(Z < 16 ? 6 : 4))) void tomo_gather_k(
     TomoArgs a, int zper) {
   using S = GatherShape<SPARSE>;
-  __shared__ float2 tile[kRP * kRP * kRZP];
+  static_assert(Z == 16 || Z == 8 || Z == 4, "rows of a product: slices, slices x (re, im), two patch rows of these");
+  constexpr int ZP = Z + 1;                  // pitch of a staged point
+  constexpr int NA = 1 + Z / 16;             // products of a step: re and im, or both in one
+  constexpr int P = Z == 4 ? 2 : 1;          // patch rows in a product: r and r + NS
+  constexpr int NS = (S::NR + P - 1) / P;
+  __shared__ float2 tile[kRP * kRP * ZP];
   const int4 it = a.items[xcd_tile(blockIdx.x, gridDim.x)];
   const int z0 = blockIdx.y * zper, nzb = min(zper, a.nz - z0);
   const int n2 = 2 * a.n;
@@ -200,35 +210,15 @@ __global__ __launch_bounds__(64 * kGatherWaves) __attribute__((amdgpu_waves_per_
   const int gy0 = it.y * kRG, gx0 = it.x * kRG;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int q = lane & 15, kk = lane >> 4;
-  constexpr int PP = kRP / 2;  // pairs of points of a row (2n is even: the wrap splits none)
-  constexpr int NT = 64 * kGatherWaves, NP = kRZ * kRP * PP;
-  static_assert(NP % NT == 0, "every thread stages the same number of pairs");
-  f32x4 v[NP / NT];
-#pragma unroll
-  for (int k = 0; k < NP / NT; ++k) {
-    const int idx = threadIdx.x + k * NT, zr = idx / PP, x = (idx - zr * PP) * 2;
-    const int z = zr / kRP, r = zr - z * kRP;
-    int gr = gy0 + r, gx = gx0 + x;
-    gr -= gr >= n2 ? n2 : 0;
-    gx -= gx >= n2 ? n2 : 0;
-    v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (z < nzb) v[k] = *reinterpret_cast<const f32x4u*>(a.G + (z0 + z) * plane + (int64_t)gr * n2 + gx);
-  }
-#pragma unroll
-  for (int k = 0; k < NP / NT; ++k) {
-    const int idx = threadIdx.x + k * NT, zr = idx / PP, x = (idx - zr * PP) * 2;
-    const int z = zr / kRP, r = zr - z * kRP;
-    float2* t = tile + (r * kRP + x) * kRZP + z;
-    t[0] = make_float2(v[k].x, v[k].y);
-    t[kRZP] = make_float2(v[k].z, v[k].w);
-  }
-  __syncthreads();
-  // SPARSE: one group, whose rows the wavefronts share (wv, wv + 8, wv + 16)
-  for (int g = SPARSE ? it.z : it.z + wv; g < it.z + it.w; g += SPARSE ? 1 : kGatherWaves) {
+  // the lane's sample of a group and its weights
+  int s = 0, cell = 0;
+  float wx[S::NX], wy[S::NR];
+  auto group = [&](int g) {
     const int2 en = a.ge[16 * g + q];
-    const int cell = a.gc[g], s = en.x, ox = en.y & 0xff, oy = en.y >> 8;
+    cell = a.gc[g];
+    s = en.x;
+    const int ox = en.y & 0xff, oy = en.y >> 8;
     const float* w = a.wt + (int64_t)max(s, 0) * (2 * kWRow);
-    float wx[S::NX], wy[S::NR];
 #pragma unroll
     for (int j = 0; j < S::NX; ++j) {
       const int i = 4 * j + kk - ox;  // tap
@@ -239,54 +229,114 @@ __global__ __launch_bounds__(64 * kGatherWaves) __attribute__((amdgpu_waves_per_
       const int i = (SPARSE ? wv + r * kGatherWaves : r) - oy;
       wy[r] = !SPARSE || (i >= 0 && i < kTL) ? w[kWRow + 3 + i] : 0.f;
     }
-    const float2* base = tile + (((cell >> 8) * kCellY * kRP) + (cell & 0xff) * kCellX + kk) * kRZP + q;
-    if constexpr (SPARSE) base += wv * kRP * kRZP;
-    f32x4 re{0.f, 0.f, 0.f, 0.f}, im{0.f, 0.f, 0.f, 0.f};
+  };
+  if constexpr (SPARSE) group(it.z);  // in flight with the staging
+  constexpr int PP = kRP / 2;  // pairs of points of a row (2n is even: the wrap splits none)
+  constexpr int NT = 64 * kGatherWaves, NP = Z * kRP * PP, NL = (NP + NT - 1) / NT;
+  f32x4 v[NL];
 #pragma unroll
-    for (int r = 0; r < S::NR; ++r) {
-      f32x4 ar{0.f, 0.f, 0.f, 0.f}, ai{0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < NL; ++k) {
+    const int idx = threadIdx.x + k * NT, zr = idx / PP, x = (idx - zr * PP) * 2;
+    const int z = zr / kRP, r = zr - z * kRP;
+    int gr = gy0 + r, gx = gx0 + x;
+    gr -= gr >= n2 ? n2 : 0;
+    gx -= gx >= n2 ? n2 : 0;
+    if (z < nzb) v[k] = *reinterpret_cast<const f32x4u*>(a.G + (z0 + z) * plane + (int64_t)gr * n2 + gx);
+  }
+#pragma unroll
+  for (int k = 0; k < NL; ++k) {
+    const int idx = threadIdx.x + k * NT, zr = idx / PP, x = (idx - zr * PP) * 2;
+    const int z = zr / kRP, r = zr - z * kRP;
+    float2* t = tile + (r * kRP + x) * ZP + z;
+    if (z >= nzb) continue;  // rows of the product that no slice has stay as they are
+    t[0] = make_float2(v[k].x, v[k].y);
+    t[ZP] = make_float2(v[k].z, v[k].w);
+  }
+  __syncthreads();
+  // SPARSE: one group, whose rows the wavefronts share (wv, wv + 8, wv + 16)
+  for (int g = SPARSE ? it.z : it.z + wv; g < it.z + it.w; g += SPARSE ? 1 : kGatherWaves) {
+    if constexpr (!SPARSE) group(g);
+    constexpr int RS = SPARSE ? kGatherWaves : 1;  // from one of the wavefront's rows to the next
+    const int at = (((cell >> 8) * kCellY + (SPARSE ? wv : 0)) * kRP + (cell & 0xff) * kCellX + kk) * ZP;
+    // the lane's float of a point (Z < 16); of a second patch row that is not
+    // there the first is read again, and not added
+    const int lf = P == 1 ? q : (q & 7) + (q >> 3) * 2 * NS * RS * kRP * ZP;
+    const int lf1 = S::NR % P == 0 ? lf : q & 7;  // in the last step
+    f32x4 sum[NA], acc[NS][NA];
+#pragma unroll
+    for (int c = 0; c < NA; ++c) sum[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < NS; ++r) {
+#pragma unroll
+      for (int c = 0; c < NA; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < S::NX; ++j) {
-        const float2 b = base[((SPARSE ? r * kGatherWaves : r) * kRP + 4 * j) * kRZP];
-        ar = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, wx[j], ar, 0, 0, 0);
-        ai = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, wx[j], ai, 0, 0, 0);
+        const float2* t = tile + at + (r * RS * kRP + 4 * j) * ZP;
+        if constexpr (Z == 16) {
+          const float2 b = t[q];
+          acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, wx[j], acc[r][0], 0, 0, 0);
+          acc[r][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, wx[j], acc[r][1], 0, 0, 0);
+        } else {
+          const float b = reinterpret_cast<const float*>(t)[r + 1 < NS ? lf : lf1];
+          acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(b, wx[j], acc[r][0], 0, 0, 0);
+        }
       }
-      re += wy[r] * ar;
-      im += wy[r] * ai;
+#pragma unroll
+      for (int c = 0; c < NA; ++c) sum[c] += wy[r] * acc[r][c];
     }
-    // rows 4 (l / 16) + i are slices, columns q samples; c1d[t] = -(-1)^t, and t
-    // has the parity of s (n is even)
+    if constexpr (P == 2) {  // the upper lanes hold rows NS and on, which follow the others in the sum
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[0][i] = __shfl(sum[0][i], lane & 31, 64);
+#pragma unroll
+      for (int r = NS; r < S::NR; ++r) sum[0] += wy[r] * acc[r - NS][0];
+    }
+    // rows 4 (l / 16) + i of the products are slices (below 16 re and im of two
+    // of them), columns q samples; c1d[t] = -(-1)^t, and t has the parity of s (n
+    // is even)
+    constexpr int ZL = P * Z / 4;  // slices of a lane
     auto store = [&](int i, float2 o) {
-      const int z = 4 * kk + i;
-      if (s >= 0 && z < nzb) a.Sh[(int64_t)s * a.nz + z0 + z] = (s & 1) ? o : make_float2(-o.x, -o.y);
+      const int z = ZL * (P == 1 ? kk : kk & 1) + i;
+      if (s >= 0 && z < nzb && (P == 1 || kk >= 2)) a.Sh[(int64_t)s * a.nz + z0 + z] = (s & 1) ? o : make_float2(-o.x, -o.y);
     };
     if constexpr (SPARSE) {
       __syncthreads();  // every wavefront has read the tile
       f32x4* part = reinterpret_cast<f32x4*>(tile);
-      part[(2 * wv) * 64 + lane] = re;
-      part[(2 * wv + 1) * 64 + lane] = im;
+#pragma unroll
+      for (int c = 0; c < NA; ++c) part[(NA * wv + c) * 64 + lane] = sum[c];
       __syncthreads();
-      if (wv >= 4) return;
-      const float* p = reinterpret_cast<const float*>(tile) + 4 * lane + wv;
+      if (wv >= ZL) return;
+      const float* p = reinterpret_cast<const float*>(tile) + 4 * lane + (Z == 16 ? wv : 2 * wv);
       float2 o = make_float2(0.f, 0.f);
 #pragma unroll
-      for (int k = 0; k < kGatherWaves; ++k) o = cadd(o, make_float2(p[2 * k * 256], p[(2 * k + 1) * 256]));
+      for (int k = 0; k < kGatherWaves; ++k)
+        o = cadd(o, make_float2(p[NA * k * 256], Z == 16 ? p[(NA * k + 1) * 256] : p[NA * k * 256 + 1]));
       store(wv, o);
       return;
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) store(i, make_float2(re[i], im[i]));
+      for (int i = 0; i < ZL; ++i)
+        store(i, Z == 16 ? make_float2(sum[0][i], sum[NA - 1][i]) : make_float2(sum[0][2 * i], sum[0][2 * i + 1]));
     }
   }
 }
 
 static hipError_t launch_gather(const TomoArgs& a, hipStream_t st) {
-  const int zblocks = (a.nz + kRZ - 1) / kRZ, zper = (a.nz + zblocks - 1) / zblocks;
-  const dim3 grid((unsigned)a.nitems, (unsigned)zblocks);
-  if (a.sparse)
-    hipLaunchKernelGGL((tomo_gather_k<true>), grid, dim3(64 * kGatherWaves), 0, st, a, zper);
-  else
-    hipLaunchKernelGGL((tomo_gather_k<false>), grid, dim3(64 * kGatherWaves), 0, st, a, zper);
+  // eights where an odd number of them holds the slab (20 slices of 512^2, 200
+  // angles: 223 us in two sixteens, 196 in three eights)
+  const int Z = a.nz <= 4 ? 4 : ((a.nz + 7) / 8) & 1 ? 8 : 16;
+  const int zblocks = (a.nz + Z - 1) / Z, zper = (a.nz + zblocks - 1) / zblocks;
+  const dim3 grid((unsigned)a.nitems, (unsigned)zblocks), block(64 * kGatherWaves);
+#define HTAMD_GATHER(SPARSE, Z) hipLaunchKernelGGL((tomo_gather_k<SPARSE, Z>), grid, block, 0, st, a, zper)
+  if (a.sparse) {
+    if (Z == 4) HTAMD_GATHER(true, 4);
+    if (Z == 8) HTAMD_GATHER(true, 8);
+    if (Z == 16) HTAMD_GATHER(true, 16);
+  } else {
+    if (Z == 4) HTAMD_GATHER(false, 4);
+    if (Z == 8) HTAMD_GATHER(false, 8);
+    if (Z == 16) HTAMD_GATHER(false, 16);
+  }
+#undef HTAMD_GATHER
   return hipGetLastError();
 }
 

@@ -276,3 +276,19 @@ def test_slices_keep_their_bits_in_any_slab(gpu, n, ntheta):
         assert torch.equal(t.R(y), full[0][:, z0:z0 + k]), k
         assert torch.equal(t.RT(s), full[1][z0:z0 + k]), k
         assert torch.equal(t.fbp(s), full[2][z0:z0 + k]), k
+
+
+@pytest.mark.parametrize("n,ntheta", [(64, 5), (64, 200), (50, 20), (10, 300)])
+def test_R_of_few_slices_has_the_bits_of_a_slab(gpu, n, ntheta):
+    """The gather's forms for up to 4, 8 and 16 slices, over cells and over
+    regions (few angles), form each sample's sum in one order."""
+    from holotomocupy_amd import Tomo
+    print(f"[case] R of few slices n={n} ntheta={ntheta}", flush=True)
+    rng = np.random.default_rng(n + ntheta)
+    nz = 32
+    t = Tomo(n, nz, angles(ntheta), 0)
+    for real in (False, True):
+        x = dev(data(rng, (nz, n, n), real))
+        full = t.R(x)
+        for k in (1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 24):
+            assert torch.equal(t.R(x[3:3 + k].contiguous()), full[:, 3:3 + k]), (real, k)

@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256) void bs_interp_rows_k(BsArgs<T> a) {
 // with magnification >= 1 through LDS (adj_tile_add), else (wider brackets) each
 // thread walks the candidates of its kAtR rows of one column.  Each output sums
 // detector rows in ascending order either way.
-// 384 planes of 256^2: 269 us walking the candidates -> 141 us (both planes
+// 384 planes of 256^2: 271 us walking the candidates -> 124 us (both planes
 // move once: 78 us at the card's copy rate).
 template <typename T>
 __global__ __launch_bounds__(256) void bs_adjoint_k(BsArgs<T> a) {

@@ -124,8 +124,14 @@ __device__ __forceinline__ float2 block_sum2(float2 v) {
 // coefficient rows that weigh them, so an output costs about 5 reads for x and
 // 4 for y, all from LDS.  Walking the candidates per output row group read each
 // pixel some 28 times through the L1, eight predicated loads to a row, and waited
-// for each row; here all loads of a tile are in flight together (without that the
-// tile form measured 247 us against the walk's 269, with it 141).
+// for each row; here all loads of a tile are in flight together.
+// The larger the magnification, the fewer pixels reach a tile and the more the
+// weights cost (candidates are tried in FP64): they are formed once for a tile,
+// rows by one wavefront and columns by another, and a tile that no pixel reaches
+// ends at once.  384 planes of 256^2: walking the candidates 271 us at
+// magnification 1, 149 at 1.5, 121 at 1.92, 81 at 4; tiles with the column
+// weights formed by every wavefront and all 44 x 76 pixels asked for 136, 125,
+// 119 and 108; so 124, 99, 94 and 80.
 // Magnification >= 1 leaves at most 4 pixels with a weight along each axis,
 // consecutive ones within the first 8 of the bracket; taps that are not there
 // read a zeroed slot, so nothing else enters the sums, which run in the order of
@@ -137,8 +143,8 @@ template <typename TO>
 struct AdjTile {
   TO g[kAtNY][kAtNX + 1];    // the last column of each row stays zero
   TO tmp[kAtNY + 1][kAtX];   // x sums; the last row stays zero
-  float wy[kAtY][4];
-  int fy[kAtY];
+  float wy[kAtY][4], wx[kAtX][4];
+  int fy[kAtY], fx[kAtX];
 };
 
 // 4 consecutive weights w with which index i collects pixels f .. f + 3 (f = -1: none)
@@ -147,13 +153,14 @@ __device__ __forceinline__ int bs_adj_taps(int i, int npix, int npsi, float mb, 
   bs_candidates(i, npix, npsi, mb, r, lo, hi);
 #pragma unroll
   for (int j = 0; j < 4; ++j) w[j] = 0.0f;
+  hi = min(hi, lo + 7);
 #pragma unroll 2
-  for (int k = 0; k < 8; ++k) {
-    const float v = lo + k <= hi ? bs_reach(bs_pos(lo + k, npix, npsi, mb, r), i) : 0.0f;
-    if (f < 0 && v != 0.0f) f = lo + k;
+  for (int p = lo; p <= hi; ++p) {
+    const float v = bs_reach(bs_pos(p, npix, npsi, mb, r), i);
+    if (f < 0 && v != 0.0f) f = p;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (f >= 0 && lo + k == f + j) w[j] = v;
+      if (f >= 0 && p == f + j) w[j] = v;
   }
   return f;
 }
@@ -176,7 +183,8 @@ __device__ __forceinline__ void adj_tile_add(AdjTile<TO>& s, int ix0, int iy0, i
   bs_candidates(iy0, nz, nzpsi, mb, ry, ylo, unused);
   bs_candidates(min(iy0 + kAtY, nzpsi) - 1, nz, nzpsi, mb, ry, unused, yhi);
   const int ncol = min(xhi - xlo + 1, kAtNX), nrow = min(yhi - ylo + 1, kAtNY);
-  __syncthreads();  // the last tile's sums have been read
+  if (ncol <= 0 || nrow <= 0) return;  // the whole workgroup: nothing reaches the tile
+  __syncthreads();                     // the last tile's sums have been read
   // (a position that is not finite gives a bracket anywhere: only pixels that
   // exist are read, and those with a weight do).  All loads are issued before
   // the first is stored.
@@ -186,27 +194,51 @@ __device__ __forceinline__ void adj_tile_add(AdjTile<TO>& s, int ix0, int iy0, i
     const unsigned ty = (unsigned)ylo + r, tx = (unsigned)xlo + k;
     return r < nrow && k < ncol && tx < (unsigned)n && ty < (unsigned)nz ? load((int)ty, (int)tx) : vzero<TO>();
   };
+  // rows beyond the first 24 and columns beyond 64 are there at magnifications
+  // below about 1.9 and 1.1
+  constexpr int NH = 6;
+  const bool tall = nrow > 4 * NH, wide = ncol > 64;
 #pragma unroll
-  for (int i = 0; i < NR; ++i) v[i] = at(wv + 4 * i, c);
+  for (int i = 0; i < NH; ++i) v[i] = at(wv + 4 * i, c);
+  if (tall) {
 #pragma unroll
-  for (int i = 0; i < NL; ++i) v[NR + i] = at((t + 256 * i) / NE, 64 + (t + 256 * i) % NE);
-  if (t < kAtY) {
-    float w[4];
-    s.fy[t] = iy0 + t < nzpsi ? bs_adj_taps(iy0 + t, nz, nzpsi, mb, ry, w) : -1;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) s.wy[t][j] = iy0 + t < nzpsi ? w[j] : 0.0f;
+    for (int i = NH; i < NR; ++i) v[i] = at(wv + 4 * i, c);
   }
+  if (wide) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) v[NR + i] = at((t + 256 * i) / NE, 64 + (t + 256 * i) % NE);
+  }
+  // the tile's weights, once: rows by the first wavefront, columns by the second
+  if (t < kAtX + kAtX && (wv || t < kAtY)) {
+    const int i = wv ? ix0 + c : iy0 + t;
+    const bool in = i < (wv ? npsi : nzpsi);
+    float w[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    int f = -1;
+    if (in) f = wv ? bs_adj_taps(i, n, npsi, mb, rx, w) : bs_adj_taps(i, nz, nzpsi, mb, ry, w);
+    float* dst = wv ? s.wx[c] : s.wy[t];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dst[j] = w[j];
+    (wv ? s.fx[c] : s.fy[t]) = f;
+  }
+#pragma unroll
+  for (int i = 0; i < NH; ++i) s.g[wv + 4 * i][c] = v[i];
+  if (tall) {
+#pragma unroll
+    for (int i = NH; i < NR; ++i) s.g[wv + 4 * i][c] = v[i];
+  }
+  if (wide) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      if (t + 256 * i < kAtNY * NE) s.g[(t + 256 * i) / NE][64 + (t + 256 * i) % NE] = v[NR + i];
+  }
+  __syncthreads();
   float wx[4];
-  const int fx = bs_adj_taps(min(ix0 + c, npsi - 1), n, npsi, mb, rx, wx);
   int ox[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) ox[j] = wx[j] != 0.0f ? fx - xlo + j : kAtNX;
-#pragma unroll
-  for (int i = 0; i < NR; ++i) s.g[wv + 4 * i][c] = v[i];
-#pragma unroll
-  for (int i = 0; i < NL; ++i)
-    if (t + 256 * i < kAtNY * NE) s.g[(t + 256 * i) / NE][64 + (t + 256 * i) % NE] = v[NR + i];
-  __syncthreads();
+  for (int j = 0; j < 4; ++j) {
+    wx[j] = s.wx[c][j];
+    ox[j] = wx[j] != 0.0f ? s.fx[c] - xlo + j : kAtNX;
+  }
   for (int r = wv; r < nrow; r += 4) {
     TO sum = vzero<TO>();
 #pragma unroll

@@ -210,3 +210,22 @@ def test_Sadj_tiles(gpu, real, n, npsi, nz, nzpsi):
     out2 = g.Sadj(dev(s), dev(r), dev(m)).cpu().numpy()
     assert np.array_equal(np.isfinite(out2), ~reach)
     assert np.array_equal(out2[~reach], out[~reach])
+
+
+@pytest.mark.parametrize("real", [False, True])
+@pytest.mark.parametrize("n,npsi,nz,nzpsi", [(200, 130, 150, 98), (300, 320, 40, 32)])
+def test_Sadj_tiles_by_magnification(gpu, real, n, npsi, nz, nzpsi):
+    """Magnifications around those at which a tile needs its last rows (about
+    1.9) and columns (about 1.1), and tiles that no detector pixel reaches."""
+    from holotomocupy_amd import Shift
+    print(f"[case] Sadj by magnification n={n} npsi={npsi} real={real}", flush=True)
+    rng = np.random.default_rng(n + nz)
+    dt = "float32" if real else "complex64"
+    m = np.array([1.0, 1.04, 1.07, 1.1, 1.13, 1.6, 1.7, 1.75, 1.8, 1.85, 1.9, 2.0, 6.0, 6.0], np.float32)
+    r = rng.uniform(-4, 4, (len(m), 2)).astype(np.float32)
+    r[-1] = (4 * nz, 4 * n)  # past the plane
+    g, o = Shift(n, npsi, nz, nzpsi, dt), osh.Shift(n, npsi, nz, nzpsi, dt)
+    s = data(rng, (len(m), nz, n), real)
+    out, ref = g.Sadj(dev(s), dev(r), dev(m)).cpu().numpy(), o.Sadj(s, r, m)
+    for b in range(len(m)):
+        assert np.linalg.norm(out[b] - ref[b]) <= REL_TOL * np.linalg.norm(ref[b]), b

@@ -493,8 +493,13 @@ constexpr int kHeavyTile = 128;
 constexpr int kLongTile = 512;  // from here more wavefronts share a long list (few slices)
 constexpr int kParts = 16, kQuarters = 4;
 constexpr int kBatch = 4;  // steps of four samples taken together
+// A grid of more than this, half the Infinity Cache, is not kept in the L2: the
+// samples' slices, which the next tiles read, are (RT of 256 slices of 256^2, 384
+// angles 787 -> 736 us; 100 slices, 64 angles 174 -> 162).  A smaller one is, for
+// the column pass (16 slices of 512^2, 16 angles 105 -> 92 us).
+constexpr int64_t kKeepGrid = 128 << 20;
 
-template <int VEC, int U, int NW, int SUBS>
+template <int VEC, int U, int NW, int SUBS, bool KEEP>
 __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
   constexpr int NA = 2 * VEC * U;  // accumulators: float columns of 16 slices
   constexpr int PX = 4 * NW;       // points of a workgroup's row
@@ -707,11 +712,12 @@ __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
   if (skipped[t >> 1]) return;
   for (int r = threadIdx.x / TR; r < 4 * (z1 - z0); r += 64 * NW / TR) {
     const int zl = r >> 2, y = r & 3;
-    // not kept in the L2: the samples' slices, which the next tiles read, are
-    // (787 -> 736 us)
-    __builtin_nontemporal_store(
-        *reinterpret_cast<const f32x4u*>(out + zl * ZS + y * PX + t * 2),
-        reinterpret_cast<f32x4u*>(a.G + (z0 + zl) * plane + (int64_t)(gy + y) * n2 + tx0 * 4 + t * 2));
+    const f32x4u v = *reinterpret_cast<const f32x4u*>(out + zl * ZS + y * PX + t * 2);
+    auto* d = reinterpret_cast<f32x4u*>(a.G + (z0 + zl) * plane + (int64_t)(gy + y) * n2 + tx0 * 4 + t * 2);
+    if constexpr (KEEP)
+      *d = v;
+    else
+      __builtin_nontemporal_store(v, d);
   }
 }
 
@@ -722,8 +728,14 @@ static hipError_t launch_grid_gather(const TomoArgs& a, hipStream_t st) {
   const int nt = a.n / 2;
   const int zblocks = (a.nz + 63) / 64, zper = ((a.nz + zblocks - 1) / zblocks + 1) / 2 * 2;
   auto grid = [&](int nw) { return dim3((unsigned)(a.nheavy + (nt + nw - 1) / nw * nt), (unsigned)zblocks); };
-#define HTAMD_GRID(VEC, U, NW, SUBS) \
-  hipLaunchKernelGGL((tomo_grid_k<VEC, U, NW, SUBS>), grid(NW), dim3(64 * NW), 0, st, a, zper)
+  const bool keep = (int64_t)a.nz * 4 * a.n * a.n * (int64_t)sizeof(float2) <= kKeepGrid;
+#define HTAMD_GRID(VEC, U, NW, SUBS)                                                                             \
+  do {                                                                                                           \
+    if (keep)                                                                                                    \
+      hipLaunchKernelGGL((tomo_grid_k<VEC, U, NW, SUBS, true>), grid(NW), dim3(64 * NW), 0, st, a, zper);        \
+    else                                                                                                         \
+      hipLaunchKernelGGL((tomo_grid_k<VEC, U, NW, SUBS, false>), grid(NW), dim3(64 * NW), 0, st, a, zper);       \
+  } while (0)
   const bool parts = a.parts == kParts;
   if (zper <= 16 && parts)
     HTAMD_GRID(1, 1, 16, 1);

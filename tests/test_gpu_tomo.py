@@ -292,3 +292,18 @@ def test_R_of_few_slices_has_the_bits_of_a_slab(gpu, n, ntheta):
         full = t.R(x)
         for k in (1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 24):
             assert torch.equal(t.R(x[3:3 + k].contiguous()), full[:, 3:3 + k]), (real, k)
+
+
+@pytest.mark.parametrize("n,nz,ntheta", [(256, 64, 90), (256, 65, 90), (512, 16, 12), (512, 17, 12), (340, 36, 40),
+                                         (340, 37, 40)])
+def test_RT_on_either_side_of_the_kept_grid(gpu, n, nz, ntheta):
+    """Grids of at most and more than 128 MiB are stored in two ways: a slab's
+    slices have the bits of slices alone."""
+    from holotomocupy_amd import Tomo
+    print(f"[case] RT kept grid n={n} nz={nz}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n + nz)
+    d = torch.randn((ntheta, nz, n), dtype=torch.complex64, device="cuda", generator=g)
+    t = Tomo(n, nz, angles(ntheta), 0)
+    full = t.RT(d)
+    for z in (0, nz // 2, nz - 1):
+        assert torch.equal(t.RT(d[:, z:z + 1].contiguous())[0], full[z]), z

@@ -16,7 +16,6 @@
 //   K4 object:  gather-form Sadj summed over distances              -> dpsi
 // then the B-spline prefilter of dpsi and two small deterministic reductions.
 #include <algorithm>
-#include <climits>
 
 #include "bh_common.hpp"
 

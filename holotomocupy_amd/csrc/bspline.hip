@@ -6,7 +6,6 @@
 // Sampling point of output pixel (tx, ty) of angle b (cuda_kernels.py:172-181):
 //   x = (m_b (tx - n/2) - r_b[1] + (m_b - 1)/2) + npsi/2      (same for y, r_b[0])
 // taps floor(x) + j, j = -1..2, weights phi(dx - j), phi = 6 * cubic B-spline.
-#include <climits>
 
 #include "htamd_bspline.hpp"
 #include "htamd_internal.hpp"

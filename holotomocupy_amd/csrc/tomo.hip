@@ -34,7 +34,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(8)));  // an odd slice count leaves rows 8-byte aligned
 
 struct TomoArgs {
-  int n = 0, nz = 0, ntheta = 0, m = 0;
+  int n = 0, nz = 0, ntheta = 0;
   const float* phi = nullptr;      // [n, n] deapodisation (mask and scale included)
   const float2* tw2 = nullptr;     // twiddles of length 2n
   const float2* tw1 = nullptr;     // twiddles of length n
@@ -1086,8 +1086,6 @@ using namespace htamd;
 
 struct htamd_tomo_plan {
   int64_t n = 0, ntheta = 0;
-  int m = 0;
-  double mu = 0.0;
   int device = -1;
   float* phi = nullptr;
   float2* tw2 = nullptr;
@@ -1149,13 +1147,13 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
   p->ntheta = ntheta;
   // eps, mu, m (tomo.py:14-16)
   const double eps = 1e-3;
-  p->mu = -std::log(eps) / (2.0 * (double)n * (double)n);
-  p->m = (int)std::ceil(2.0 * n / M_PI * std::sqrt(-p->mu * std::log(eps) + (p->mu * n) * (p->mu * n) / 4.0));
-  if (2 * p->m + 1 != kTL) {  // 4 for every n: the kernels are built for 9x9 windows
+  const double mu = -std::log(eps) / (2.0 * (double)n * (double)n);
+  const int m = (int)std::ceil(2.0 * n / M_PI * std::sqrt(-mu * std::log(eps) + (mu * n) * (mu * n) / 4.0));
+  if (2 * m + 1 != kTL) {  // 4 for every n: the kernels are built for 9x9 windows
     delete p;
     return fail(HTAMD_ERR_UNSUPPORTED, "tomo_plan_create: gridding half-width is not 4");
   }
-  const int L = 2 * p->m + 1;
+  const int L = 2 * m + 1;
   const int64_t S = ntheta * n, n2 = 2 * n;
   if (S * L * L > (int64_t)INT32_MAX) {
     delete p;
@@ -1168,7 +1166,7 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
   // weights exp(-pi^2/mu d^2) (x) and pi/mu exp(-pi^2/mu d^2) (y).
   std::vector<int2> tb((size_t)S);
   std::vector<float> wt((size_t)(2 * kWRow * S), 0.0f);
-  const double cy = M_PI / p->mu, cx = -M_PI * M_PI / p->mu, inv2n = 1.0 / (double)n2;
+  const double cy = M_PI / mu, cx = -M_PI * M_PI / mu, inv2n = 1.0 / (double)n2;
   for (int64_t k = 0; k < ntheta; ++k) {
     const double th = (double)(float)theta[k];
     const double c = std::cos(th), sn = std::sin(th);
@@ -1176,8 +1174,8 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
       const int64_t si = k * n + t;
       const double x0 = (double)(t - n / 2) / (double)n * c;
       const double y0 = -(double)(t - n / 2) / (double)n * sn;
-      const int bx = (int)std::floor((double)n2 * x0) - p->m;
-      const int by = (int)std::floor((double)n2 * y0) - p->m;
+      const int bx = (int)std::floor((double)n2 * x0) - m;
+      const int by = (int)std::floor((double)n2 * y0) - m;
       tb[(size_t)si] = make_int2(bx, by);
       float* w = &wt[(size_t)(2 * kWRow * si)];
       for (int i = 0; i < L; ++i) {
@@ -1276,7 +1274,7 @@ int htamd_tomo_plan_create(int64_t n, int64_t ntheta, const double* theta, const
     const double dy = -0.5 + (double)i / (double)n;
     for (int64_t j = 0; j < n; ++j) {
       const double dx = -0.5 + (double)j / (double)n;
-      double v = std::exp(p->mu * (double)(n * n) * (dx * dx + dy * dy)) * (double)(1 - n % 4);
+      double v = std::exp(mu * (double)(n * n) * (dx * dx + dy * dy)) * (double)(1 - n % 4);
       v *= (mask ? mask[i * n + j] : 1.0) / ((double)n * std::sqrt((double)n * (double)ntheta));
       phi[(size_t)(i * n + j)] = (float)v;
     }
@@ -1357,7 +1355,6 @@ static int tomo_run(const htamd_tomo_plan* p, bool adjoint, const void* in, int 
   a.n = (int)p->n;
   a.nz = (int)nz;
   a.ntheta = (int)p->ntheta;
-  a.m = p->m;
   a.phi = p->phi;
   a.wt = p->wt;
   a.tp = p->tp;

@@ -434,8 +434,9 @@ class Rec(BHLoop):
     def _tomo_slab(self):
         """Slices per R / RT call on device-resident arrays: as many as keep the
         Radon workspace (htamd_tomo_workspace_size: 6 nobj^2 + ntheta nobj
-        complex64 per slice) within 4 GiB, a multiple of 32 (the RT gather's
-        slice block) when that many fit, and at least nchunk."""
+        complex64 per slice) within 4 GiB, a multiple of 32 when that many
+        fit (the gridding products take 16 to 64 slices at a time), and at
+        least nchunk.  A slice's result does not depend on its slab."""
         per_slice = 8 * (6 * self.nobj * self.nobj + self.ntheta * self.nobj)
         slab = max(1, (4 << 30) // per_slice)
         if slab >= 32:

@@ -62,7 +62,7 @@ __device__ __forceinline__ int64_t row_tile(int64_t bid, int64_t nblocks, int nd
 // 256^2, 3 distances, 64 angles 637 -> 618 us).
 constexpr int kXcdGroups = 8;
 
-constexpr int64_t kNumCu = 256, kCuLds = 160 * 1024;
+constexpr int64_t kCuLds = 160 * 1024;
 
 // Whether `blocks` workgroups, of which a CU holds per_cu (at most waves_cu
 // by their registers, and what their LDS leaves room for), run in whole

@@ -6,6 +6,7 @@
 namespace htamd {
 
 constexpr int kNumXcd = 8;  // MI355X: 256 CUs in 8 XCDs, workgroups dealt round-robin
+constexpr int64_t kNumCu = 256;
 
 __host__ __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __host__ __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }

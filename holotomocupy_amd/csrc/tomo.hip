@@ -726,7 +726,12 @@ __global__ __launch_bounds__(64 * NW) void tomo_grid_k(TomoArgs a, int zper) {
 // the last slices).
 static hipError_t launch_grid_gather(const TomoArgs& a, hipStream_t st) {
   const int nt = a.n / 2;
-  const int zblocks = (a.nz + 63) / 64, zper = ((a.nz + zblocks - 1) / zblocks + 1) / 2 * 2;
+  // Blocks of 64 slices, or of 16 where long lists have fewer workgroups than the
+  // chip has CUs (RT of 40 slices of 32^2, 1200 angles 250 -> 96 us).
+  const bool parts = a.parts == kParts;
+  const int64_t blocks64 = (a.nz + 63) / 64;
+  const int zmax = parts && nt * nt * blocks64 <= kNumCu ? 16 : 64;
+  const int zblocks = (a.nz + zmax - 1) / zmax, zper = ((a.nz + zblocks - 1) / zblocks + 1) / 2 * 2;
   auto grid = [&](int nw) { return dim3((unsigned)(a.nheavy + (nt + nw - 1) / nw * nt), (unsigned)zblocks); };
   const bool keep = (int64_t)a.nz * 4 * a.n * a.n * (int64_t)sizeof(float2) <= kKeepGrid;
 #define HTAMD_GRID(VEC, U, NW, SUBS)                                                                             \
@@ -736,7 +741,6 @@ static hipError_t launch_grid_gather(const TomoArgs& a, hipStream_t st) {
     else                                                                                                         \
       hipLaunchKernelGGL((tomo_grid_k<VEC, U, NW, SUBS, false>), grid(NW), dim3(64 * NW), 0, st, a, zper);       \
   } while (0)
-  const bool parts = a.parts == kParts;
   if (zper <= 16 && parts)
     HTAMD_GRID(1, 1, 16, 1);
   else if (zper <= 16)

@@ -307,3 +307,20 @@ def test_RT_on_either_side_of_the_kept_grid(gpu, n, nz, ntheta):
     full = t.RT(d)
     for z in (0, nz // 2, nz - 1):
         assert torch.equal(t.RT(d[:, z:z + 1].contiguous())[0], full[z]), z
+
+
+@pytest.mark.parametrize("n,ntheta", [(8, 200), (32, 160)])
+def test_slices_keep_their_bits_on_small_grids(gpu, n, ntheta):
+    """Grids of fewer tiles than CUs take slabs in blocks of 16 slices, and of
+    64 where there are enough blocks: RT of a slice is the same in all."""
+    from holotomocupy_amd import Tomo
+    print(f"[case] RT small grid n={n} ntheta={ntheta}", flush=True)
+    rng = np.random.default_rng(n)
+    nz = 1100 if n == 8 else 150
+    t = Tomo(n, nz, angles(ntheta), 0)
+    d = dev(data(rng, (ntheta, nz, n), False))
+    full = t.RT(d)
+    for k in (1, 17, 40, 64, 65, 66):
+        assert torch.equal(t.RT(d[:, 5:5 + k].contiguous()), full[5:5 + k]), k
+    for z in (0, nz - 1):
+        assert torch.equal(t.RT(d[:, z:z + 1].contiguous())[0], full[z]), z

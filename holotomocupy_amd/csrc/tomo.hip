@@ -241,6 +241,7 @@ __global__ __launch_bounds__(64 * kGatherWaves) __attribute__((amdgpu_waves_per_
     int gr = gy0 + r, gx = gx0 + x;
     gr -= gr >= n2 ? n2 : 0;
     gx -= gx >= n2 ? n2 : 0;
+    if constexpr (Z == 16) v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (z < nzb) v[k] = *reinterpret_cast<const f32x4u*>(a.G + (z0 + z) * plane + (int64_t)gr * n2 + gx);
   }
 #pragma unroll
@@ -248,7 +249,7 @@ __global__ __launch_bounds__(64 * kGatherWaves) __attribute__((amdgpu_waves_per_
     const int idx = threadIdx.x + k * NT, zr = idx / PP, x = (idx - zr * PP) * 2;
     const int z = zr / kRP, r = zr - z * kRP;
     float2* t = tile + (r * kRP + x) * ZP + z;
-    if (z >= nzb) continue;  // rows of the product that no slice has stay as they are
+    if (Z < 16 && z >= nzb) continue;  // rows of the product that no slice has stay as they are
     t[0] = make_float2(v[k].x, v[k].y);
     t[ZP] = make_float2(v[k].z, v[k].w);
   }

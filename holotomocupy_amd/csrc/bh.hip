@@ -498,7 +498,7 @@ __global__ __launch_bounds__(kRowThreads) void bh_adj_rows_k(BhArgs a) {
 // walking the candidates of each output.  Each output sums over detector rows in
 // ascending order and the distances in order.
 // 16 angles of 1024^2 from 4 distances of 2048^2: 512 us walking the candidates
-// -> 306 us; 48 angles of 256^2 from 2 distances 69 -> 39 us.
+// -> 252 us; 48 angles of 256^2 from 2 distances 69 -> 33 us.
 template <typename TO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void bh_sadj_k(BhArgs a, TO* __restrict__ dpsi, int tiles_x,
                                                  int tiles_y) {
@@ -706,7 +706,7 @@ static RowShape row_shape(int64_t n, int64_t nz, int64_t ndist, int64_t npsi, in
 // K3 splits the angles into groups (see there) where one angle's row units are
 // fewer than kAdjSplitBelow workgroups and do not fill rounds of the chip
 // (registers admit three workgroups per CU, their LDS often two).  256^2, 2
-// distances, 48 angles (64 workgroups): 815 -> 149 us and 5 us for
+// distances, 48 angles (64 workgroups): 815 -> 142 us and 5 us for
 // bh_prb_final_k; the whole gradient at 1024^2, 2 distances, 32 angles: with
 // 512^2 objects (1024 workgroups in rounds of 768) 2500 -> 2320 us, with 1024^2
 // ones (two rounds of 512, not split) split 1979 -> 2002 us.

@@ -521,9 +521,9 @@ static BhhLayout bhh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* s
 // rows of a workgroup stay within 64 KiB of dynamic LDS.
 constexpr int64_t kHessDynBudget = 65536;
 // The chain kernel's angles are independent: they are split over workgroups until there are about this many, unless
-// one angle's row units are one whole round.  Pair form at 256^2, 4 distances, 32 angles: 781 -> 541 us in all;
-// 1024^2, 16 angles, 512^2 objects (2048 workgroups): 4533 -> 4427 us; equal form at 1024^2, 1 distance, 22 angles,
-// 1024^2 objects (512, one round): split 1600 -> 1623 us.
+// one angle's row units are one whole round.  Pair form at 256^2, 4 distances, 48 angles: 1503 -> 1008 us in all; at
+// 1024^2, 16 angles, 512^2 objects (2048 workgroups) 4448 and 4419 us, within what runs differ by; equal form at
+// 1024^2, 1 distance, 22 angles, 1024^2 objects (512, one round): split 1600 -> 1623 us.
 constexpr int64_t kHessBlocks = 4096;
 
 template <int N, typename TO, int MODE>

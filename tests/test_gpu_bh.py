@@ -321,16 +321,17 @@ def test_gradient_workspace_holds_no_second_work_field(gpu, n, nobj, ndist, B):
     assert BHGradient(rec).workspace_bytes(B) <= base + max(0, groups * slot - obj) + 8 * 256
 
 
-@pytest.mark.parametrize("accumulate", [False, True])
-def test_probe_runs_over_several_windows(gpu, accumulate):
+@pytest.mark.parametrize("accumulate,nobj", [(False, 32), (True, 32), (False, 160)])
+def test_probe_runs_over_several_windows(gpu, accumulate, nobj):
     """More groups of angles than their sums have slots (18 of 43 angles, 21
     groups): a run that begins in one window of groups and ends in the next, and
-    runs of one angle on both sides, give the bits of each run alone."""
-    print(f"[case] probe runs over windows accumulate={accumulate}", flush=True)
+    runs of one angle on both sides, give the bits of each run alone.  Also with
+    object rows that are too wide to be staged (and room for all groups)."""
+    print(f"[case] probe runs over windows accumulate={accumulate} nobj={nobj}", flush=True)
     from holotomocupy_amd.bh import BHGradient
     runs = (1,) * 10 + (30,) + (1,) * 3
     B, k = sum(runs), len(runs)
-    rec, cas, x, v, w, d = make_problem(False, n=64, nobj=32, ndist=2, B=B, seed=65)
+    rec, cas, x, v, w, d = make_problem(False, n=64, nobj=nobj, ndist=2, B=B, seed=65)
     xd, dd = dev(x), torch.from_numpy(d).cuda()
     bh = BHGradient(rec)
     mag = rec.eff_demagnifications[:B].contiguous()

@@ -722,10 +722,17 @@ constexpr int64_t kFwdBlocks = 4096;
 
 // Slots of the group sums.  One run of angles has a quarter as many groups as
 // angles, runs of five angles 2/5, and only shorter ones more: such calls take
-// several windows.  Up to eight slots, and as many as the object gradient has
-// room for (it is formed after the group sums have been used), cost nothing.
-static int64_t adj_slots(int64_t nang, int64_t slot_bytes, int64_t dpsi_bytes) {
-  return std::min(nang, std::max({(int64_t)8, (2 * nang + 4) / 5, dpsi_bytes / slot_bytes}));
+// several windows, and so do those whose windows are kAdjWindow workgroups
+// without that (a slot is 16 KiB for each of a group's workgroups, so this
+// bounds the slots' bytes by 256 MiB whatever the angles).  As many slots as the
+// object gradient has room for cost nothing: it is formed after they are used.
+// Workspace of 128 angles of 1024^2, 2 distances, 512^2 objects 4835 -> 2688 MB
+// (as without groups), 8.07-8.11 ms either way; 600 angles of 256^2, 4 distances
+// 3151 -> 1893 MB, 6.50 and 6.40 ms.
+constexpr int64_t kAdjWindow = 8192;
+static int64_t adj_slots(int64_t nang, int64_t blocks, int64_t slot_bytes, int64_t dpsi_bytes) {
+  const int64_t most = std::max((int64_t)8, (kAdjWindow + blocks - 1) / blocks);
+  return std::min(nang, std::max({(int64_t)8, std::min(most, (2 * nang + 4) / 5), dpsi_bytes / slot_bytes}));
 }
 
 static BhLayout bh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* sp, int64_t nang) {
@@ -744,7 +751,7 @@ static BhLayout bh_layout(const htamd_prop_plan* pp, const htamd_shift_plan* sp,
   int64_t room = nang * plane * osz;
   if (nang > kAdjGroup && adj_split(pp->n, pp->nz, pp->ndist, sp->npsi, osz)) {  // up to one group: the same sum either way
     const int64_t slot = pp->ndist * field * 8;
-    L.slots = adj_slots(nang, slot, room);
+    L.slots = adj_slots(nang, row_shape(pp->n, pp->nz, pp->ndist, sp->npsi, osz, true).blocks, slot, room);
     room = std::max(room, L.slots * slot);
   }
   off += align256(room);

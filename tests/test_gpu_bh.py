@@ -307,17 +307,19 @@ def test_tab_call_with_scattered_probes(gpu):
         assert torch.equal(one["proj"][0], gproj[b]) and torch.equal(one["pos"][0], gpos[b]), b
 
 
-@pytest.mark.parametrize("n,nobj,ndist,B", [(256, 256, 2, 48), (256, 128, 2, 48), (128, 128, 3, 9), (64, 48, 2, 300)])
+@pytest.mark.parametrize("n,nobj,ndist,B", [(256, 256, 2, 48), (256, 128, 2, 48), (128, 128, 3, 9), (64, 48, 2, 300),
+                                            (512, 64, 2, 500)])
 def test_gradient_workspace_holds_no_second_work_field(gpu, n, nobj, ndist, B):
     """The group sums of the split row pass take the room of the object gradient,
     which is formed after them, and beyond it at most two slots to five angles
-    (at least eight) where the work field has one per angle."""
+    (at least eight) where the work field has one per angle, nor more than a
+    window of 8192 workgroups needs."""
     print(f"[case] gradient workspace n={n} nobj={nobj} ndist={ndist} B={B}", flush=True)
     from holotomocupy_amd.bh import BHGradient
     rec = make_problem(False, n=n, nobj=nobj, ndist=ndist, B=1, seed=64)[0]
     obj, slot = B * nobj * nobj * 8, ndist * n * n * 8
     base = 2 * obj + B * slot + B * ndist * n * 16  # coefficients, object gradient, work field, partial sums
-    groups = min(B, max(8, -(-2 * B // 5)))
+    groups = min(B, max(8, min(-(-2 * B // 5), -(-8192 * 2048 // (ndist * n * n)))))
     assert BHGradient(rec).workspace_bytes(B) <= base + max(0, groups * slot - obj) + 8 * 256
 
 
@@ -358,3 +360,30 @@ def test_probe_runs_over_several_windows(gpu, accumulate, nobj):
         assert torch.equal(one["prb"], gprb[i]), i
         assert torch.equal(one["proj"], gproj[sl]) and torch.equal(one["pos"], gpos[sl]), i
         st += m
+
+
+def test_one_run_over_two_windows(gpu):
+    """80 angles of one probe at 1024^2: 20 groups in windows of 15.  Object and
+    position gradients are those of the angles by fives, the probe gradient their
+    sum (up to its rounding)."""
+    print("[case] one run over two windows", flush=True)
+    from types import SimpleNamespace
+    from holotomocupy_amd.rec import Rec
+    n, nobj, B = 1024, 64, 80
+    rec = Rec(SimpleNamespace(energy=17.1, detector_pixelsize=1.4760147601476e-6 * 4, focustodetectordistance=1.217,
+                              z1=np.array([5.110]) * 1e-3, ndist=1, ntheta=B, nz=n, n=n, nzobj=nobj, nobj=nobj,
+                              obj_dtype="complex64", rho=[1, 0.5, 0.2]))
+    g = torch.Generator(device="cuda").manual_seed(66)
+    c = lambda *s: torch.randn(s, dtype=torch.complex64, device="cuda", generator=g)  # noqa: E731
+    x = {"prb": 1 + 0.1 * c(1, n, n), "proj": 0.1 * c(B, nobj, nobj),
+         "pos": torch.randn((B, 1, 2), device="cuda", generator=g)}
+    d = 1 + 0.1 * torch.rand((B, 1, n, n), device="cuda", generator=g)
+    one = {k: torch.zeros_like(t) for k, t in x.items()}
+    rec.gradients_fused(x, one, d)
+    part = {k: torch.zeros_like(t) for k, t in x.items()}
+    for st in range(0, B, 5):
+        sl = slice(st, st + 5)
+        rec.gradients_fused({"prb": x["prb"], "proj": x["proj"][sl], "pos": x["pos"][sl]},
+                            {"prb": part["prb"], "proj": part["proj"][sl], "pos": part["pos"][sl]}, d[sl], st=st)
+    assert torch.equal(one["proj"], part["proj"]) and torch.equal(one["pos"], part["pos"])
+    assert rel(one["prb"], part["prb"].cpu().numpy()) < 1e-6
